@@ -1,0 +1,90 @@
+"""The packed kernel (4/6/2; two diagonals per lane and register) at the sizes
+where its tiling can go wrong: end diagonals at the edges of chunks (116 own
+diagonals, 6 copies at each end) and of lanes, sequence lengths around its
+16-base words, every window and wave count, sequences expanded in LDS (short
+ones) and packed (long ones in narrow windows), plain and queue-fed.  Scores
+are whole numbers and must equal the oracle's."""
+import random
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print(f"\n[gpu] {msg}", flush=True)
+
+
+def seq(rng, n):
+    return "".join(rng.choice("ACGT") for _ in range(n))
+
+
+def edited(rng, s, k):
+    s = list(s)
+    for _ in range(k):
+        i = rng.randrange(len(s))
+        c = rng.random()
+        if c < 0.34:
+            s[i] = rng.choice("ACGT")
+        elif c < 0.67:
+            s.insert(i, rng.choice("ACGT"))
+        else:
+            del s[i]
+    return "".join(s)
+
+
+def check(aligner, oracle, pairs, wf_length):
+    want, _, _ = oracle.wfa_batch(pairs, 4, 6, 2)
+    b = aligner.batch(pairs)
+    say(f"plain wf_length={wf_length}, {len(pairs)} pairs")
+    got, _ = aligner.align_plain(b, wf_length)
+    assert (got == want).all(), np.nonzero(got != want)[0][:5]
+    say("batched")
+    got, _ = aligner.align_batched(b)
+    assert (got == want).all(), np.nonzero(got != want)[0][:5]
+
+
+@pytest.mark.parametrize("wf_length,base,gaps", [
+    (64, 40, (0, 1, 5, 14)),
+    (128, 100, (0, 1, 30, 50)),
+    (256, 150, (57, 58, 59, 63, 64, 65, 90)),
+    (512, 300, (57, 58, 115, 116, 117, 121, 122, 173, 174, 175, 200)),
+    (1024, 500, (57, 58, 173, 174, 231, 232, 233, 347, 348, 400)),
+    (2000, 1500, (115, 116, 231, 232, 700)),
+    (4096, 2500, (115, 116, 117, 463, 464, 465, 1200)),
+    (8192, 3500, (927, 928, 929, 2500)),
+    (16384, 4500, (1855, 1856, 1857, 3500)),
+])
+def test_end_diagonal_at_chunk_edges(aligner, oracle, wf_length, base, gaps):
+    """One long gap (either way) puts the end diagonal at a chosen place."""
+    rng = random.Random(wf_length)
+    pairs = []
+    for g in gaps:
+        for _ in range(2):
+            p = seq(rng, base)
+            i = rng.randrange(base)
+            t = edited(rng, p[:i] + seq(rng, g) + p[i:], 3)
+            pairs += [(p, t), (t, p)]
+    check(aligner, oracle, pairs, wf_length)
+
+
+@pytest.mark.parametrize("length", [1, 15, 16, 17, 31, 33, 63, 64, 65, 127, 128, 129, 255, 257, 1000])
+def test_lengths_around_words(aligner, oracle, length):
+    rng = random.Random(length)
+    pairs = [(p, edited(rng, p, 1 + length // 12) or "A") for p in (seq(rng, length) for _ in range(24))]
+    pairs += [(seq(rng, length), seq(rng, rng.randint(1, length))) for _ in range(8)]
+    pairs += [("A" * length, "A" * max(1, length - 3)), ("AC" * length, "CA" * length), ("A" * length, "T" * length)]
+    check(aligner, oracle, pairs, 2 * length + 400)
+
+
+@pytest.mark.parametrize("length,edits,wf_length", [(6000, 12, 128), (9000, 30, 512), (16001, 40, 512), (31990, 60, 1024),
+                                                    (31990, 300, 4096)])
+def test_long_accurate_reads(aligner, oracle, length, edits, wf_length):
+    """Long runs (extended by the whole wave) on packed sequences, up to the
+    longest the kernel takes."""
+    rng = random.Random(length + edits)
+    pairs = [(p, edited(rng, p, edits)) for p in (seq(rng, length) for _ in range(4))]
+    p = seq(rng, 700) * (length // 700)          # repeats: many cells extend at once
+    pairs.append((p, edited(rng, p, edits // 2)))
+    check(aligner, oracle, pairs, wf_length)

@@ -517,25 +517,53 @@ int tsu_host::ml_waves(const tsu_ctx* ctx, int32_t W, int32_t max_len) {
     return nw;
 }
 
-// Register kernels when the penalties and the capacity allow: one wave for
-// up to 512 diagonals, 2-16 waves of 8 chunks for up to 8192, 4-16 waves of
-// 16 chunks (older M scores in LDS) for up to 16384 (and the two sequences
-// fit in LDS).
+// Waves per CU below which the packed kernel keeps its sequences packed in
+// LDS instead of expanded (a compare takes 8 instead of 20 vector
+// instructions, at nine times the LDS).  Measured on 30,000 pairs of
+// 100-20,000 bp at 1-15%: 12 waves 73.4 ms, 16 73.9, 8 76.9, always
+// expanded 81.5, never 89.8; 10,000 pairs of 10,240 bp in 512 diagonals take
+// 0.573 ms packed and 1.83 expanded (3 waves per CU).
+constexpr int64_t kPkMinWaves = 12;
+
+// Packed kernel (scaled penalties 2/3/1, sequences of at most 32000 bases):
+// the window for capacity W, its waves and chunks, and whether the sequences
+// are expanded in LDS.  The plain form's windows decide which pairs fit:
+// 64 * 2^j diagonals up to 1,024, then 4,096 on; the other forms (queue-fed),
+// which re-run a pair that overflows, take 2,048 first.
+bool tsu_host::use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh) {
+    if (!tsu_host::fixed_242(ctx) || W > 16 * 1024 || max_len > kPackedMaxLen) return false;
+    Shape r = sh;
+    r.pk = true;
+    r.reg_c = 9;
+    r.nw = 1;
+    r.win = 64;
+    while (r.win < W) r.win *= 2;
+    if (r.win <= 1024) {
+        r.reg_c = r.win <= 128 ? 1 : r.win == 256 ? 3 : r.win == 512 ? 5 : 9;
+    } else {
+        if (!r.queue) r.win = std::max(r.win, 4096);
+        r.nw = r.win / 1024;
+    }
+    KArgs a = base_args(ctx);
+    a.seq_words = seq_words_for(ctx, max_len);
+    r.expand = true;
+    r.expand = ctx->max_lds / tsu::lds_bytes(r, a) * r.nw >= kPkMinWaves;
+    if (tsu::lds_bytes(r, a) > ctx->max_lds) return false;
+    sh = r;
+    return true;
+}
+
+// Register kernels when the penalties and the capacity allow: the packed
+// kernel for sequences of at most 32000 bases; beyond, offsets in 32 bits:
+// one wave for up to 512 diagonals, 2-16 waves of 8 chunks for up to 8192
+// (and the two sequences fit in LDS).
 static void use_register_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh) {
     if (max_len > tsu_host::max_seq_len(ctx)) return;  // the register kernels stage both sequences in LDS
+    if (tsu_host::use_packed_kernel(ctx, W, max_len, sh)) return;
     Shape r = sh;
     if (int c = tsu_host::reg_chunks(ctx, W)) {
         r.reg_c = c;
         r.nw = 1;
-        // the int16 LDS ring variant (doubled offsets fit int16 up to 16000
-        // bases) measured faster only with 8 chunks on short sequences; with
-        // narrower windows or long, extend-heavy pairs its ring traffic costs
-        // more than the DPP moves it saves
-        r.lring = c == 8 && max_len <= 4096;
-    } else if (int nwl = tsu_host::ml_waves(ctx, W, max_len)) {
-        r.reg_c = 16;
-        r.nw = nwl;
-        r.dbl = max_len <= tsu::kMlDblMaxLen;
     } else if (int nw = tsu_host::reg_waves(ctx, W)) {
         r.reg_c = 8;
         r.nw = nw;
@@ -628,9 +656,9 @@ extern "C" int tsu_align_plain(tsu_ctx* ctx, tsu_batch* b, int32_t wf_length, in
     }
     int launches = 1;
     const bool clean = lowest >= 0;
-    if (!clean && (sh.reg_c == 16 || sh.lring || (sh.two_piece && sh.reg_c))) {
-        // the kernels with an int16 LDS ring stop past their score limit with
-        // an overflow status: such pairs get the LDS kernel at the same
+    if (!clean && sh.two_piece && sh.reg_c) {
+        // the 2-piece register kernel stops past its score limit with an
+        // overflow status: such pairs get the LDS-ring kernel at the same
         // capacity, so whether a pair fits depends on the capacity and not on
         // that limit (the re-run's launch counts in the wall time)
         const double r0 = now_ms();
@@ -638,17 +666,8 @@ extern "C" int tsu_align_plain(tsu_ctx* ctx, tsu_batch* b, int32_t wf_length, in
         for (int32_t i = 0; i < b->n; ++i)
             if (scores[i] == TSU_EKOVERFLOW) again.push_back(i);
         if (!again.empty()) {
-            Shape s2{default_waves(W), b->max_len <= 32000, true, false, true};
-            s2.fixed_242 = sh.fixed_242;
-            if (sh.two_piece) {  // the 2-piece LDS-ring kernel
-                s2.nw = 1;
-                s2.two_piece = true;
-            }
-            tsu_host::place_sequences(ctx, s2, b->max_len);
-            KArgs a2 = base_args(ctx);
-            a2.W = W;
-            a2.seq_words = seq_words_for(ctx, b->max_len);
-            if (tsu::lds_bytes(s2, a2) > ctx->max_lds) { s2.lds_ring = false; s2.nw = 16; }
+            Shape s2{1, b->max_len <= 32000, true, false, true};
+            s2.two_piece = true;
             DevBuf<int32_t> d_order;
             HIPCHK(d_order.alloc(again.size()), "hipMalloc (order)");
             HIPCHK(hipMemcpy(d_order.p, again.data(), again.size() * sizeof(int32_t), hipMemcpyHostToDevice), "hipMemcpy (order)");
@@ -864,8 +883,7 @@ static int run_probe(tsu_ctx* ctx, tsu_batch* b, std::vector<int32_t>& ids, int3
     pa.probe_out = d_prog.p;
     Shape ps{1, max_len <= 32000, true, false, true};
     ps.fixed_242 = true;
-    ps.reg_c = 8;
-    ps.probe = true;
+    tsu_host::probe_shape(max_len, ps);
     HIPCHK(hipMemcpyAsync(d_order, ids.data(), ids.size() * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream),
            "hipMemcpyAsync (order)");
     int r = run_shape(ctx, io_of(b), ps, 512, d_order, (int32_t)ids.size(), max_len, 0, &pa, kms);

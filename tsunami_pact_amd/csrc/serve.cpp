@@ -224,8 +224,7 @@ int64_t plan_flight(tsu_server* s, Slot& sl, int32_t W_entry, int* status) {
         lp.W = 512;
         lp.sh = Shape{1, lp.max_len <= 32000, true, false, true};
         lp.sh.fixed_242 = true;
-        lp.sh.reg_c = 8;
-        lp.sh.probe = true;
+        tsu_host::probe_shape(lp.max_len, lp.sh);
     } else {
         lp.W = W_entry > 0 ? std::min(W_entry, full) : W0;
         lp.sh = tsu_host::batched_shape(ctx, lp.W, lp.max_len, W_entry > 0 ? 0 : waves);

@@ -143,6 +143,13 @@ int reg2p_chunks(const tsu_ctx* ctx, int32_t W, int32_t max_len);
 // ring) for capacity W and sequences up to max_len (0: not eligible).
 int ml_waves(const tsu_ctx* ctx, int32_t W, int32_t max_len);
 
+// Longest sequence the packed kernel takes: its offsets, and one past the
+// last one of a text with its padding, are exact in 16 bits.
+constexpr int32_t kPackedMaxLen = 32000;
+// Packed kernel for capacity W and sequences up to max_len: fills in sh, or
+// returns false where it does not apply.
+bool use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh);
+
 // Probe of the batched and served forms: the single-wave register kernel
 // runs a pair up to kProbeCap scaled scores (its 512-diagonal window holds
 // the range that far), and the furthest h + v it reached gives the capacity
@@ -154,6 +161,13 @@ constexpr int32_t kProbeCap = 240;
 constexpr double kProbeMargin = 1.1;
 constexpr double kProbeMarginServed = 1.2;
 int32_t probe_capacity(const tsu_ctx* ctx, const tsu_pair& pr, int32_t progress, double margin = kProbeMargin);
+// The probe's kernel: one wave, 512 diagonals.
+inline void probe_shape(int32_t max_len, Shape& sh) {
+    sh.probe = true;
+    sh.pk = max_len <= kPackedMaxLen;
+    sh.reg_c = sh.pk ? 5 : 8;
+    sh.win = 512;
+}
 // Pairs of a length bucket are probed when the register kernels take them
 // (their sequences, up to max_len bases, fit in LDS) and the bucket's first
 // capacity (W) needs several waves.

@@ -94,6 +94,9 @@ struct Shape {
     bool dbl = false;        // 16-chunk kernel with doubled offsets (sequences up to kMlDblMaxLen bases)
     bool probe = false;      // single-wave register kernel stopping at KArgs::probe_cap
     bool gseq = false;       // LDS kernel reading the sequences from HBM (too long for LDS; int32 offsets)
+    bool pk = false;         // packed kernel: nw waves of reg_c chunks of 128 diagonals, two per register
+    bool expand = false;     // packed kernel with the sequences expanded in LDS
+    int win = 0;             // packed kernel: the window's width in diagonals (KArgs::W of the launch)
     int reg_e = 0;           // 2-piece register kernel: 10 e1 + e2 after the gcd (11, 21 or 31)
 };
 

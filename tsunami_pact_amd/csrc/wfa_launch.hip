@@ -20,6 +20,8 @@ KernelFn pick_regmw(const Shape& sh);
 int regmw_exchange_words(int nw);
 KernelFn pick_regml(const Shape& sh);
 int regml_exchange_words(int nw);
+KernelFn pick_pk(const Shape& sh);
+int64_t lds_bytes_pk(const Shape& sh, const KArgs& a);
 KernelFn pick_2p(const Shape& sh);
 int64_t lds_bytes_2p(const Shape& sh, const KArgs& a);
 
@@ -42,6 +44,7 @@ int64_t ring_bytes(const Shape& sh, int32_t W, int32_t rm, int32_t ri) {
 
 int64_t lds_bytes(const Shape& sh, const KArgs& a) {
     if (sh.two_piece) return lds_bytes_2p(sh, a);
+    if (sh.pk) return lds_bytes_pk(sh, a);
     if (sh.reg_c > 0) {
         // sequences + misc (one wave), + the edge exchange area (several waves
         // of 8 chunks), + the exchange area and the int16 M ring (16 chunks)
@@ -57,6 +60,7 @@ int64_t lds_bytes(const Shape& sh, const KArgs& a) {
 
 static KernelFn pick(const Shape& sh) {
     if (sh.two_piece) return pick_2p(sh);
+    if (sh.pk) return pick_pk(sh);
     if (sh.reg_c > 0) return sh.nw == 1 ? pick_reg(sh) : sh.reg_c == 16 ? pick_regml(sh) : pick_regmw(sh);
     switch (sh.nw) {
     case 1: return pick_nw1(sh);
@@ -119,7 +123,9 @@ int occupancy(const Shape& sh, int64_t lds, int* blocks_per_cu) {
     return 0;
 }
 
-int launch_wfa(const Shape& sh, const KArgs& a, int64_t grid, void* stream) {
+int launch_wfa(const Shape& sh, const KArgs& args, int64_t grid, void* stream) {
+    KArgs a = args;
+    if (sh.pk) a.W = sh.win;  // the packed kernel's windows are wider than the capacity asked for
     KernelFn f = pick(sh);
     if (!f) return (int)hipErrorInvalidValue;
     if (grid <= 0) return 0;

@@ -20,15 +20,6 @@ KernelFn pick_reg(const Shape& sh) {
         default: return nullptr;
         }
     }
-    if (sh.lring) {
-        switch (sh.reg_c) {
-        case 1: return sh.queue ? wfa_reg1l_kernel<1, true> : wfa_reg1l_kernel<1, false>;
-        case 2: return sh.queue ? wfa_reg1l_kernel<2, true> : wfa_reg1l_kernel<2, false>;
-        case 4: return sh.queue ? wfa_reg1l_kernel<4, true> : wfa_reg1l_kernel<4, false>;
-        case 8: return sh.queue ? wfa_reg1l_kernel<8, true> : wfa_reg1l_kernel<8, false>;
-        default: return nullptr;
-        }
-    }
     if (sh.probe) return sh.reg_c == 8 && sh.queue ? wfa_reg_kernel<8, 2, 3, 1, true, true> : nullptr;
     switch (sh.reg_c) {
     case 1: return sh.queue ? wfa_reg_kernel<1, 2, 3, 1, true> : wfa_reg_kernel<1, 2, 3, 1, false>;
