@@ -2,8 +2,8 @@
 where its tiling can go wrong: end diagonals at the edges of chunks (116 own
 diagonals, 6 copies at each end) and of lanes, sequence lengths around its
 16-base words, every window and wave count, sequences expanded in LDS (short
-ones) and packed (long ones in narrow windows), plain and queue-fed.  Scores
-are whole numbers and must equal the oracle's."""
+ones) and packed (long ones in narrow windows), plain, queue-fed and with backtrace records.  Scores
+and CIGARs are whole numbers and must equal the oracle's."""
 import random
 
 import numpy as np
@@ -35,7 +35,7 @@ def edited(rng, s, k):
 
 
 def check(aligner, oracle, pairs, wf_length):
-    want, _, _ = oracle.wfa_batch(pairs, 4, 6, 2)
+    want, ops, _ = oracle.wfa_batch(pairs, 4, 6, 2, cigar=True)
     b = aligner.batch(pairs)
     say(f"plain wf_length={wf_length}, {len(pairs)} pairs")
     got, _ = aligner.align_plain(b, wf_length)
@@ -43,6 +43,11 @@ def check(aligner, oracle, pairs, wf_length):
     say("batched")
     got, _ = aligner.align_batched(b)
     assert (got == want).all(), np.nonzero(got != want)[0][:5]
+    say("CIGARs")
+    got, cig, _ = aligner.align_cigar(b)
+    assert (got == want).all(), np.nonzero(got != want)[0][:5]
+    bad = [i for i in range(len(pairs)) if cig[i] != oracle.rle(ops[i])]
+    assert not bad, bad[:5]
 
 
 @pytest.mark.parametrize("wf_length,base,gaps", [
@@ -88,3 +93,14 @@ def test_long_accurate_reads(aligner, oracle, length, edits, wf_length):
     p = seq(rng, 700) * (length // 700)          # repeats: many cells extend at once
     pairs.append((p, edited(rng, p, edits // 2)))
     check(aligner, oracle, pairs, wf_length)
+
+
+def test_extensions_longer_than_a_record_holds(aligner, oracle):
+    """Runs of 4,094 to 12,000 matches: a record holds lengths below 4,095,
+    the others are in the list behind the records."""
+    rng = random.Random(8)
+    pairs = []
+    for n in (4093, 4094, 4095, 4096, 4097, 8191, 12000):
+        p, q = seq(rng, n), seq(rng, 300)
+        pairs += [(q + "A" + p + "C" + q, q + "T" + p + "G" + q), (p + q, p + "ACGTAC" + q), ("A" * n + q, "A" * (n + 3) + q)]
+    check(aligner, oracle, pairs, 512)

@@ -504,19 +504,6 @@ int tsu_host::reg_waves(const tsu_ctx* ctx, int32_t W) {
     return nw;
 }
 
-// Capacities above this use the 16-chunk waves with the int16 LDS M ring
-// rather than 8-chunk waves with the whole ring in registers: measured
-// faster from 1,025 diagonals on (the 4-wave, neighbour-synchronised
-// instance fits 5 pairs per CU), slower at 850.
-constexpr int32_t kMlMinCapacity = 1024;
-
-int tsu_host::ml_waves(const tsu_ctx* ctx, int32_t W, int32_t max_len) {
-    if (!tsu_host::fixed_242(ctx) || W <= kMlMinCapacity || W > 16 * 1024 || max_len > 32000) return 0;
-    int nw = 4;
-    while (1024 * nw < W) nw *= 2;
-    return nw;
-}
-
 // Waves per CU below which the packed kernel keeps its sequences packed in
 // LDS instead of expanded (a compare takes 8 instead of 20 vector
 // instructions, at nine times the LDS).  Measured on 30,000 pairs of
@@ -1417,21 +1404,22 @@ static int copy_to_host(tsu_ctx* ctx, void* dst, const void* src, size_t bytes, 
 
 namespace {
 
-// Chunks of the single-wave recording kernel for capacity W (0: none): the
-// register windows of up to 512 diagonals, and 1024 (16 chunks), which only
-// the recording instance takes.
-int bt_reg_chunks(const tsu_ctx* ctx, int32_t W) {
-    if (int c = tsu_host::reg_chunks(ctx, W)) return c;
-    return tsu_host::fixed_242(ctx) && W <= 1024 ? 16 : 0;
+// The packed kernel as a recorder: with one wave per pair it takes sequences
+// of up to 16,000 bases (longer pairs of a narrow window go to the LDS kernel
+// where their scores are known, else to a window of two waves).
+constexpr int32_t kRecordOneWaveMaxLen = 16000;
+bool use_packed_recorder(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh) {
+    Shape r = sh;
+    if (!tsu_host::use_packed_kernel(ctx, W, max_len, r) || (r.nw == 1 && max_len > kRecordOneWaveMaxLen)) return false;
+    sh = r;
+    return true;
 }
 
-// Kernel family of a CIGAR launch at capacity W for a pair of length len
-// and scaled score s: 1 the single-wave register kernel, 2 + waves the
-// 16-chunk kernel, 0 the LDS kernel.
-int bt_family(const tsu_ctx* ctx, int32_t W, int32_t len, int64_t s) {
-    if (bt_reg_chunks(ctx, W) > 0 && len <= 16000 && s <= 16000) return 1;
-    if (int nw = tsu_host::ml_waves(ctx, W, len)) return 2 + nw;
-    return 0;
+// Kernel family of a CIGAR launch at capacity W for a pair of length len:
+// the waves of the packed kernel, or 0 for the LDS kernel.
+int bt_family(const tsu_ctx* ctx, int32_t W, int32_t len) {
+    Shape sh{1, true, true, true, true};
+    return use_packed_recorder(ctx, W, len, sh) ? sh.nw : 0;
 }
 
 // Highest scaled score a pair of lengths (p, t) can have: min(p, t)
@@ -1594,8 +1582,10 @@ int CigarCall::launch_bt(const Shape& sh, KArgs& a, int32_t W, const std::vector
     cg->kernels |= tsu_host::kernel_bit(sh);
     void *rec = nullptr, *slo = nullptr, *soff = nullptr, *ckb = nullptr;
     HIPCHK(bt_reserve(ctx, 0, (size_t)(recs * grid) * 4, &rec), "hipMalloc (records)");
-    HIPCHK(bt_reserve(ctx, 1, (size_t)((int64_t)step_cap * grid) * 4, &slo), "hipMalloc (steps)");
-    HIPCHK(bt_reserve(ctx, 2, (size_t)((int64_t)step_cap * grid) * 8, &soff), "hipMalloc (steps)");
+    if (!sh.pk) {  // records at a place that depends on the score: a table
+        HIPCHK(bt_reserve(ctx, 1, (size_t)((int64_t)step_cap * grid) * 4, &slo), "hipMalloc (steps)");
+        HIPCHK(bt_reserve(ctx, 2, (size_t)((int64_t)step_cap * grid) * 8, &soff), "hipMalloc (steps)");
+    }
     if (sh.ck) {
         a.ck_stride = (int64_t)a.ck_cap * a.ck_bytes;
         HIPCHK(bt_reserve(ctx, 3, (size_t)(a.ck_stride * grid), &ckb), "hipMalloc (checkpoints)");
@@ -1797,7 +1787,7 @@ int CigarCall::plan_records(std::vector<RecordPlan>& plans, int64_t& runs_need) 
         for (Group& g : groups) {
             int32_t ml = 0;
             for (int32_t i : g.ids) ml = std::max(ml, std::max(b->pairs[(size_t)i].p_len, b->pairs[(size_t)i].t_len));
-            if (tsu_host::ml_waves(ctx, std::min<int32_t>(g.W, capacity_full(ml, ml)), ml) == 16) {
+            if (bt_family(ctx, std::min<int32_t>(g.W, capacity_full(ml, ml)), ml) == 16) {
                 merged.W = std::max(merged.W, g.W);
                 merged.ids.insert(merged.ids.end(), g.ids.begin(), g.ids.end());
             } else {
@@ -1827,23 +1817,12 @@ void CigarCall::plan_group(int32_t W, bool placed, std::vector<int32_t>& ids, st
         s_len = std::max(s_len, score_bound(ctx, pr.p_len, pr.t_len));
     }
     W = std::min<int32_t>(W, capacity_full(max_len, max_len));
-    // the single-wave recorder holds sequences of up to 16,000 bases:
-    // longer pairs of a narrow window take the 16-chunk kernel's narrowest
-    if (max_len > 16000 && W <= kMlMinCapacity) W = std::min<int32_t>(4 * 1024, capacity_full(max_len, max_len));
     Shape sh{default_waves(W), max_len <= 32000, true, true, true};
     sh.fixed_242 = true;
-    // the kernel's own window: 64 diagonals per chunk
-    int32_t win = 0;
-    const int c1 = bt_reg_chunks(ctx, W);
-    if (c1 > 0 && max_len <= 16000) {
-        sh.nw = 1;
-        sh.reg_c = c1;
-        sh.lring = true;
-        win = 64 * c1;
-    } else if (int nwl = tsu_host::ml_waves(ctx, W, max_len)) {
-        sh.nw = nwl;
-        sh.reg_c = 16;
-        win = 1024 * nwl;
+    int32_t win = 0;  // the kernel's own window
+    if (max_len > kRecordOneWaveMaxLen && max_len <= tsu_host::kPackedMaxLen && W <= 1024) W = 2048;
+    if (use_packed_recorder(ctx, W, max_len, sh)) {
+        win = sh.win;
     } else if (placed && W > 16 * 1024) {
         // predicted beyond every register window: straight to the launch
         // over the whole diagonal range (room in the run pool for their bound)
@@ -1858,33 +1837,33 @@ void CigarCall::plan_group(int32_t W, bool placed, std::vector<int32_t>& ids, st
     }
     // a window holding every diagonal of the longest pair never overflows
     int64_t s_cap = win >= capacity_full(max_len, max_len) ? s_len : std::min(s_len, score_for_capacity(ctx, win));
-    if (s_cap < 0 || (sh.nw == 1 && s_cap > 16000)) return;
+    if (s_cap < 0) return;
     KArgs a = base_args(ctx);
     a.W = W;
     a.seq_words = seq_words_for(ctx, max_len);
     int per_cu = 0;
     if (tsu::occupancy(sh, tsu::lds_bytes(sh, a), &per_cu) != 0 || per_cu <= 0) return;
     // the launch's state (records of every resident pair) stays within
-    // the budget: fewer steps if needed, unless that leaves less than a
-    // third of the window's scores
+    // half the budget, so that two launches' states can stand beside each
+    // other: fewer steps if needed, unless that leaves less than a third of
+    // the window's scores
     const int64_t resident = std::min<int64_t>((int64_t)per_cu * ctx->cu_count, (int64_t)ids.size());
-    const int64_t step_bytes = (int64_t)win * 4 + 12;
-    const int64_t fit = budget / (resident * step_bytes) - 2;
+    const int64_t step_bytes = 4 * (tsu_host::packed_records(sh, 1) - tsu_host::packed_records(sh, 0));
+    const int64_t fit = budget / 2 / (resident * step_bytes) - tsu_host::packed_steps(1);
     const int64_t s_win = s_cap;
     if (fit < s_cap) {
         if (fit * 3 < s_cap) return;
         s_cap = fit;
     }
-    const int32_t step_cap = (int32_t)(s_cap + 2);
-    const int64_t recs = (int64_t)step_cap * win;
-    if (sh.nw > 1) sh.dbl = max_len <= tsu::kMlDblMaxLen && s_cap <= tsu::kMlDblMaxScore;
-    const int64_t per_wg = recs * 4 + (int64_t)step_cap * 12;
+    const int32_t step_cap = tsu_host::packed_steps(s_cap);
+    const int64_t recs = tsu_host::packed_records(sh, step_cap);
+    const int64_t per_wg = recs * 4;
     // pairs of the widest window may also be walked by the launch for
     // wider pairs, beside later launches: room for their whole bound
     for (int32_t i : ids) {
         const tsu_pair& pr = b->pairs[(size_t)i];
         const int64_t sb = score_bound(ctx, pr.p_len, pr.t_len);
-        runs_need += 2 * ((win >= 16 * 1024 ? sb : std::min(s_cap + 1, sb)) / unit) + 2;
+        runs_need += 2 * ((win >= 16 * 1024 ? sb : std::min<int64_t>(step_cap, sb)) / unit) + 2;
     }
     tsu_host::order_longest_first(ids, b->pairs.data());
     plans.push_back(RecordPlan{std::move(ids), sh, a, W, max_len, step_cap, win, recs, per_wg,
@@ -1931,17 +1910,13 @@ int CigarCall::record_pass() {
         // the state of the launches after it is reserved before the wide
         // launch starts: freeing a buffer to grow it waits for the whole
         // device, so growing one later would stall them until it ends
-        size_t need[3] = {0, 0, 0};
+        size_t need = 0;
         for (size_t j = k; j < plans.size(); ++j) {
             const int64_t grid = bt_grid(plans[j].sh, plans[j].a, (int64_t)plans[j].ids.size(), plans[j].per_wg);
-            need[0] = std::max(need[0], (size_t)(plans[j].recs * grid) * 4);
-            need[1] = std::max(need[1], (size_t)((int64_t)plans[j].step_cap * grid) * 4);
-            need[2] = std::max(need[2], (size_t)((int64_t)plans[j].step_cap * grid) * 8);
+            need = std::max(need, (size_t)(plans[j].recs * grid) * 4);
         }
-        for (int i = 0; i < 3; ++i) {
-            void* p = nullptr;
-            HIPCHK(bt_reserve(ctx, i, need[i], &p), "hipMalloc (records)");
-        }
+        void* p = nullptr;
+        HIPCHK(bt_reserve(ctx, 0, need, &p), "hipMalloc (records)");
         WidePlan wp = plan_wide(wide);
         if (wp.per_wg * (int64_t)wide.size() <= budget) {
             int r = launch_wide_async(wp, wide);
@@ -2024,7 +1999,7 @@ int CigarCall::score_first_pass() {
             const tsu_pair& pr = b->pairs[(size_t)order[end]];
             const int32_t len = std::max(pr.p_len, pr.t_len);
             const int32_t si = scores[order[end]] / ctx->g;
-            const int f = bt_family(ctx, std::max<int32_t>(capacity_for_score(ctx, si), 16), len, si);
+            const int f = bt_family(ctx, std::max<int32_t>(capacity_for_score(ctx, si), 16), len);
             if (family < 0) family = f;
             else if (f != family) break;
             max_len = std::max(max_len, len);
@@ -2037,21 +2012,9 @@ int CigarCall::score_first_pass() {
         sh.fixed_242 = tsu_host::fixed_242(ctx);
         int64_t recs = 0;
         int32_t step_cap = steps;
-        const int c1 = bt_reg_chunks(ctx, W);
-        if (c1 > 0 && max_len <= 16000 && s0 <= 16000) {
-            // single-wave kernel with the int16 LDS ring: records at a fixed
-            // place per step and chunk, (s * chunks + c) * 64 + lane
-            sh.nw = 1;
-            sh.reg_c = c1;
-            sh.lring = true;
-            recs = (int64_t)steps * c1 * 64;
-        } else if (int nwl = tsu_host::ml_waves(ctx, W, max_len)) {
-            // 16-chunk multi-wave kernel: records at a fixed place per step and
-            // chunk, (s * chunks + j) * 64 + lane
-            sh.nw = nwl;
-            sh.reg_c = 16;
-            sh.dbl = max_len <= tsu::kMlDblMaxLen && s0 <= tsu::kMlDblMaxScore;
-            recs = (int64_t)steps * nwl * 16 * 64;
+        if (use_packed_recorder(ctx, W, max_len, sh)) {
+            step_cap = tsu_host::packed_steps(s0);
+            recs = tsu_host::packed_records(sh, step_cap);
         } else {
             for (int64_t s = 0; s <= s0; ++s)
                 recs += std::min<int64_t>(W, 2 * (std::max<int64_t>(0, s - ctx->os) / ctx->es + 2) + 1);
@@ -2059,11 +2022,14 @@ int CigarCall::score_first_pass() {
             tsu_host::place_sequences(ctx, sh, max_len);
             if (tsu::lds_bytes(sh, a) > ctx->max_lds) { sh.lds_ring = false; sh.nw = 16; }
         }
-        int64_t per_wg = recs * 4 + (int64_t)steps * 12 + (sh.lds_ring || sh.reg_c ? 0 : tsu::ring_bytes(sh, W, ctx->rm, ctx->ri));
-        // checkpoints instead of records when records do not fit one pair per CU
+        int64_t per_wg = recs * 4 + (sh.pk ? 0 : (int64_t)steps * 12) + (sh.lds_ring || sh.pk ? 0 : tsu::ring_bytes(sh, W, ctx->rm, ctx->ri));
+        // checkpoints instead of records when records do not fit one pair per
+        // CU (16-bit records: within half the budget, the line that 32-bit
+        // ones had at the whole of it, so a budget that bounded a call's
+        // memory to checkpoints still does)
         const bool ck = ctx->cigar_mode == TSU_CIGAR_CHECKPOINTS ||
                         (ctx->cigar_mode == TSU_CIGAR_AUTO && s0 > 0 &&
-                         per_wg * std::min<int64_t>(group_n, ctx->cu_count) > budget);
+                         per_wg * std::min<int64_t>(group_n, ctx->cu_count) > (sh.pk ? budget / 2 : budget));
         if (ck) {
             sh = Shape{std::max(4, default_waves(W)), max_len <= 32000, true, true, true};
             sh.fixed_242 = tsu_host::fixed_242(ctx);
@@ -2229,7 +2195,7 @@ uint32_t tsu_host::kernel_bit(const Shape& sh) {
     if (sh.ck) return TSU_KERNEL_LDS_CK;
     if (sh.two_piece) return sh.reg_c ? TSU_KERNEL_2P_REG : TSU_KERNEL_2P;
     if (sh.reg_c > 0 && sh.nw == 1) return TSU_KERNEL_REG1;
-    if (sh.reg_c == 16) return sh.nw <= 4 ? TSU_KERNEL_ML4 : sh.nw == 8 ? TSU_KERNEL_ML8 : TSU_KERNEL_ML16;
+    if (sh.pk) return sh.nw <= 4 ? TSU_KERNEL_ML4 : sh.nw == 8 ? TSU_KERNEL_ML8 : TSU_KERNEL_ML16;
     if (sh.reg_c > 0) return TSU_KERNEL_REG1;
     return TSU_KERNEL_LDS;
 }

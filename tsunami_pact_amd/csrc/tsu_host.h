@@ -139,16 +139,18 @@ int reg_waves(const tsu_ctx* ctx, int32_t W);
 // gcd, sequences up to 16000 bases, its M ring in LDS (0: the LDS-ring
 // 2-piece kernel).
 int reg2p_chunks(const tsu_ctx* ctx, int32_t W, int32_t max_len);
-// Waves of the 16-chunk multi-wave kernel (older M scores in an int16 LDS
-// ring) for capacity W and sequences up to max_len (0: not eligible).
-int ml_waves(const tsu_ctx* ctx, int32_t W, int32_t max_len);
-
 // Longest sequence the packed kernel takes: its offsets, and one past the
 // last one of a text with its padding, are exact in 16 bits.
 constexpr int32_t kPackedMaxLen = 32000;
 // Packed kernel for capacity W and sequences up to max_len: fills in sh, or
 // returns false where it does not apply.
 bool use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh);
+// Record words per workgroup and score steps of a packed launch that records
+// scores up to s.
+inline int32_t packed_steps(int64_t s) { return (int32_t)(s + 2 + tsu::kPackedStep); }
+inline int64_t packed_records(const Shape& sh, int32_t steps) {
+    return (int64_t)steps * sh.nw * sh.reg_c * 64 + tsu::kPackedLongWords;
+}
 
 // Probe of the batched and served forms: the single-wave register kernel
 // runs a pair up to kProbeCap scaled scores (its 512-diagonal window holds

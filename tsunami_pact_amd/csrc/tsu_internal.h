@@ -88,10 +88,8 @@ struct Shape {
     bool queue;      // persistent launch fed by a work counter
     bool fixed_242 = false;  // scaled penalties are (2, 3, 1): compile-time ring
     int reg_c = 0;           // > 0: register-resident kernel, reg_c chunks of 64 diagonals per wave (nw waves)
-    bool lring = false;      // one wave: the older M scores in an int16 LDS ring (sequences up to 16000 bases)
     bool two_piece = false;  // gap-affine 2-piece kernel (one wave per pair, rings in LDS)
     bool ck = false;         // backtrace from ring checkpoints (bt and queue set, LDS kernel)
-    bool dbl = false;        // 16-chunk kernel with doubled offsets (sequences up to kMlDblMaxLen bases)
     bool probe = false;      // single-wave register kernel stopping at KArgs::probe_cap
     bool gseq = false;       // LDS kernel reading the sequences from HBM (too long for LDS; int32 offsets)
     bool pk = false;         // packed kernel: nw waves of reg_c chunks of 128 diagonals, two per register
@@ -100,11 +98,11 @@ struct Shape {
     int reg_e = 0;           // 2-piece register kernel: 10 e1 + e2 after the gcd (11, 21 or 31)
 };
 
-// Doubled-offset 16-chunk kernel: longest sequence (2t fits int16) and the
-// highest scaled score it runs to (-32768 + 2s, the ring's NULL after s
-// scores, stays negative).
-constexpr int32_t kMlDblMaxLen = 16383;
-constexpr int32_t kMlDblMaxScore = 16383;
+// Packed kernel: scores it computes between two exchanges (it may record
+// that many scores past the end), and the words behind a workgroup's records
+// that list extensions too long for one (three words each).
+constexpr int kPackedStep = 6;
+constexpr int kPackedLongWords = 768;
 
 // Device scratch of tsu_align_batched_noalloc (a file-scope array per GPU):
 // work counters, then one queue-order entry per pair.

@@ -18,8 +18,6 @@ KernelFn pick_nw16(const Shape& sh);
 KernelFn pick_reg(const Shape& sh);
 KernelFn pick_regmw(const Shape& sh);
 int regmw_exchange_words(int nw);
-KernelFn pick_regml(const Shape& sh);
-int regml_exchange_words(int nw);
 KernelFn pick_pk(const Shape& sh);
 int64_t lds_bytes_pk(const Shape& sh, const KArgs& a);
 KernelFn pick_2p(const Shape& sh);
@@ -46,11 +44,8 @@ int64_t lds_bytes(const Shape& sh, const KArgs& a) {
     if (sh.two_piece) return lds_bytes_2p(sh, a);
     if (sh.pk) return lds_bytes_pk(sh, a);
     if (sh.reg_c > 0) {
-        // sequences + misc (one wave), + the edge exchange area (several waves
-        // of 8 chunks), + the exchange area and the int16 M ring (16 chunks)
-        // (one wave with the int16 ring: 4 misc words + 3 slots of 64*reg_c + 2 entries)
-        if (sh.nw == 1 && sh.lring) return 4ll * (2 * a.seq_words + 4) + ((3 * (64 * sh.reg_c + 2) * 2 + 3) & ~3);
-        const int ex = sh.nw == 1 ? 16 : sh.reg_c == 16 ? regml_exchange_words(sh.nw) : regmw_exchange_words(sh.nw);
+        // sequences + misc (one wave), + the edge exchange area (several waves)
+        const int ex = sh.nw == 1 ? 16 : regmw_exchange_words(sh.nw);
         return 4ll * (2 * a.seq_words + ex);
     }
     int64_t b = lds_head_bytes(a.seq_words, a.rm + 2 * a.ri, sh.nw);
@@ -61,7 +56,7 @@ int64_t lds_bytes(const Shape& sh, const KArgs& a) {
 static KernelFn pick(const Shape& sh) {
     if (sh.two_piece) return pick_2p(sh);
     if (sh.pk) return pick_pk(sh);
-    if (sh.reg_c > 0) return sh.nw == 1 ? pick_reg(sh) : sh.reg_c == 16 ? pick_regml(sh) : pick_regmw(sh);
+    if (sh.reg_c > 0) return sh.nw == 1 ? pick_reg(sh) : pick_regmw(sh);
     switch (sh.nw) {
     case 1: return pick_nw1(sh);
     case 2: return pick_nw2(sh);

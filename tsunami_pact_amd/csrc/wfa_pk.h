@@ -73,14 +73,14 @@
 #include <stdint.h>
 #include <type_traits>
 
-#include "tsu_internal.h"
+#include "wfa_bt.h"
 
 namespace tsu {
 
 using KernelFn = void (*)(KArgs);
 
 constexpr uint32_t kPkNull = 0x80008000u;
-constexpr int kPkStep = 6;          // scores between two exchanges: even, and a multiple of 3
+constexpr int kPkStep = kPackedStep;  // scores between two exchanges: even, and a multiple of 3
 constexpr int kPkDrift = 17;        // 16 bases of a first compare and one of I or X
 constexpr int kPkRenull = 128;      // exchanges; copies in LDS are one period behind at most
 static_assert(2 * (kPkRenull + 1) * kPkStep * kPkDrift < 32768, "NULL stays negative");
@@ -107,6 +107,12 @@ __device__ __forceinline__ uint32_t pk_sub(uint32_t a, uint32_t b) {
 }
 __device__ __forceinline__ uint32_t pk_mul(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, (pk_u16)(__builtin_bit_cast(pk_u16, a) * __builtin_bit_cast(pk_u16, b)));
+}
+// a * b + c; b a wave-uniform constant
+__device__ __forceinline__ uint32_t pk_mad(uint32_t a, uint32_t b, uint32_t c) {
+    uint32_t r;
+    asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
+    return r;
 }
 __device__ __forceinline__ uint32_t pk_half(uint32_t a) {  // each half >> 1
     return __builtin_bit_cast(uint32_t, (pk_u16)(__builtin_bit_cast(pk_u16, a) >> (pk_u16)1));
@@ -196,6 +202,7 @@ struct PkLayout {
     static constexpr int MISC = 0;                    // [4] queue index
     static constexpr int PG = XCH + 2 * XP;           // [NW] exchanges each wave has finished
     static constexpr int EV = PG + (NW > 1 ? NW : 0); // [1] first event, score * 4 + kind
+    static constexpr int LC = EV + 1;                 // [1] long extensions recorded
     static constexpr int WORDS = EV + 4;
 };
 
@@ -212,12 +219,117 @@ constexpr int kPkEvEnd = 0, kPkEvEdge = 1, kPkEvInternal = 3;
 constexpr int kPkNoEvent = 0x7fffffff;
 constexpr int kPkSpinCap = 1 << 20;
 
+// Backtrace records: 16 bits per cell, one coalesced 256-byte store per chunk
+// and score at ((s * NC + j) * 64 + lane) of the workgroup's region.  The
+// kernel keeps no I and D, and a cell's sources are maxima taken at their own
+// diagonal, so the gap bits sit where the gap comes from:
+//   bit 0   M[s][k] before extension is not X (ties M > D > I,
+//           common.h:67-77)
+//   bit 1   ... and not D either, so I where bit 0 is set as well
+//   bit 2   I[s+1][k+1] opens from M[s-3][k] rather than extending I[s][k]
+//   bit 3   D[s+1][k-1] opens from M[s-3][k] rather than extending D[s][k]
+//   bits 4-15  the extension's length; kPkLong and above: kPkLong, and the
+//           length in the list behind the records (score, diagonal, length)
+// The walk arrives at a cell with its offset after extension, so the length
+// gives the offset before.  16 bits per cell are half the record traffic and
+// half the state of records that hold the offset itself.
+constexpr uint32_t kPkLong = 4095;
+
+// The walk, by all lanes of a wave in step.  It is a chain of dependent
+// reads, so the records of 32 scores and 16 diagonals around the current cell
+// are loaded at once (four dwords per lane) and read from there until a step
+// leaves the block (a mismatch moves 2 scores down a diagonal, a gap 1 or 4
+// scores and one diagonal); the block of the next 32 scores on the same
+// diagonals is loaded ahead, so its round trip to memory overlaps the steps
+// through this one.  Scores are those of the penalties 2/3/1.
+template <int NC, int OWN, int HL>
+__device__ __forceinline__ int pk_walk(const uint32_t* rec, const uint32_t* longs, int n_longs, int kb, int s_max, int score,
+                                       int p, int t, const KArgs& a, int64_t* out_off, int32_t* out_n) {
+    const int lane = (int)(threadIdx.x & 63);
+    BtWalk w;
+    w.need = 2 * (int64_t)(score / 2) + 2;
+    unsigned long long b0 = 0;
+    if (lane == 0) b0 = atomicAdd(a.runs_used, (unsigned long long)w.need);
+    const uint32_t blo = __builtin_amdgcn_readfirstlane((uint32_t)b0);
+    const uint32_t bhi = __builtin_amdgcn_readfirstlane((uint32_t)(b0 >> 32));
+    w.base = (int64_t)(((uint64_t)bhi << 32) | blo);
+    if (w.base + w.need > a.runs_cap) return TSU_ECIGAR;
+    w.out = a.runs + w.base;
+    w.nr = 0;
+    w.cur_op = 4; w.cur_len = 0;
+    w.full = false;
+    w.writer = lane == 0;
+    w.k = t - p; w.off = t; w.ss = score; w.type = 0;
+    w.v = p; w.h = t;
+    w.x = 2; w.o = 3; w.e = 1;
+    int bs = -1, bd = 0, nd = 0;   // the block's top score and first dword; the next block's first dword
+    uint32_t blk[4], nxt[4];       // scores bs - lane/8 - 8 i, dword bd + lane%8; the same of bs - 32
+    auto load = [&](uint32_t (&x)[4], int ss, int d0) __attribute__((always_inline)) {
+        const int q = min(max(d0 + (lane & 7), 0), NC * OWN / 2 - 1);
+        const uint32_t* at = rec + (q / (OWN / 2)) * 64 + HL + q % (OWN / 2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = at[(int64_t)max(ss - 8 * i - (lane >> 3), 1) * NC * 64];
+    };
+    // the record of score ss (1..score) on diagonal k: false outside the window
+    auto record = [&](int ss, int k, uint32_t& r) __attribute__((always_inline)) -> bool {
+        const int d = k - kb;
+        if (ss < 1 || ss > s_max || d < 0 || d >= NC * OWN) return false;
+        const int dw = d >> 1;
+        if ((unsigned)(bs - ss) > 31u || (unsigned)(dw - bd) > 7u) {
+            if (bs > 0 && (unsigned)(bs - 32 - ss) < 8u && (unsigned)(dw - nd) < 8u) {
+                bs -= 32; bd = nd;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) blk[i] = nxt[i];
+            } else {
+                bs = ss; bd = dw - 4;
+                load(blk, bs, bd);
+            }
+            nd = dw - 4;
+            load(nxt, bs - 32, nd);
+        }
+        const int row = bs - ss, li = __builtin_amdgcn_readfirstlane(8 * (row & 7) + dw - bd);
+        const int q = __builtin_amdgcn_readfirstlane(row >> 3);
+        const uint32_t x = q == 0 ? blk[0] : q == 1 ? blk[1] : q == 2 ? blk[2] : blk[3];
+        const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)x, li);
+        r = (v >> (16 * (d & 1))) & 0xffffu;
+        return true;
+    };
+    while (w.v > 0 && w.h > 0 && w.ss > 0) {
+        uint32_t r;
+        if (w.type == 0) {
+            if (!record(w.ss, w.k, r)) return TSU_EINTERNAL;
+            int e = (int)(r >> 4);
+            if (e == (int)kPkLong) {
+                int i = 0;
+                while (i < n_longs && !((int)longs[3 * i] == w.ss && (int)longs[3 * i + 1] == w.k)) ++i;
+                if (i >= n_longs) return TSU_ECIGAR;  // the list was too short
+                e = (int)longs[3 * i + 2];
+            }
+            w.emit(0, e);
+            w.off -= e; w.v = w.off - w.k; w.h = w.off;
+            if (w.v < 0 || w.h < 0) return TSU_EINTERNAL;
+            if (w.v == 0 || w.h == 0) break;
+            if (!(r & 1u)) { w.emit(1, 1); w.ss -= 2; --w.off; --w.v; --w.h; continue; }
+            w.type = (r & 2u) ? 1 : 2;
+        }
+        if (w.type == 1) {
+            w.emit(2, 1); --w.k; --w.off;
+        } else {
+            w.emit(3, 1); ++w.k;
+        }
+        if (!record(w.ss - 1, w.k, r)) return TSU_EINTERNAL;
+        if (r & (w.type == 1 ? 4u : 8u)) { w.ss -= 4; w.type = 0; } else --w.ss;
+        w.v = w.off - w.k; w.h = w.off;
+    }
+    return bt_end(w, out_off, out_n);
+}
+
 // W is the window's width in diagonals as the host counts it (it may be less
 // than the chunks hold): the range a pair may use is
 // [kmin, kmin + W - 1], kmin = max(-W/2, -p-1), moved down where it would
 // pass t + 1; a non-NULL cell on its first or last diagonal (where that is
 // no bound of the alignment) ends the pair with TSU_EKOVERFLOW.
-template <int NW, int C, bool H, bool QUEUE, bool PROBE = false>
+template <int NW, int C, bool H, bool QUEUE, bool PROBE = false, bool BT = false>
 __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
     static_assert(NW >= 1 && NW <= 16 && C >= 1 && C <= 16, "at most 16 waves of 16 chunks");
     static_assert(!PROBE || NW == 1, "the probe runs on one wave");
@@ -243,6 +355,12 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
     const int wl = w == 0 ? NW - 1 : w - 1;  // owner of chunk j-1
     const int wr = w == NW - 1 ? 0 : w + 1;  // owner of chunk j+1
     const int poll_limit = a.poll_limit > 0 ? a.poll_limit : kPkSpinCap;
+    uint32_t* rec = nullptr;    // BT: this workgroup's records, then its long extensions
+    uint32_t* longs = nullptr;
+    if constexpr (BT) {
+        rec = a.rec_g + (int64_t)blockIdx.x * a.rec_cap;
+        longs = rec + a.rec_cap - kPackedLongWords;
+    }
 
     for (int iter = 0;; ++iter) {
         int idx;
@@ -270,7 +388,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
             sS[i] = wt;
         }
         for (int i = L::XCH + tid; i < L::WORDS; i += NT)
-            X[i] = i < L::PG ? (int32_t)kPkNull : i < L::EV ? 0 : kPkNoEvent;
+            X[i] = i < L::PG ? (int32_t)kPkNull : i == L::EV ? kPkNoEvent : 0;
         __syncthreads();
         if constexpr (H) {
             // two positions per 32-bit word: a window of 16 bases at 2i gives both
@@ -473,15 +591,42 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
             asm volatile("" : "+s"(em), "+s"(el), "+s"(eh));
             const uint32_t special = (em | el | eh) & (1u << c);
             Words q;
+            uint32_t flags = 0;  // BT: record bits 0-3 of the score in flight
+            uint32_t* rs = nullptr;  // the chunk's records of the next score (uniform)
+            if constexpr (BT) rs = rec + ((int64_t)(s0 + 1) * NC + NW * c + w) * 64;
             // the result of score s's compare, and what hangs on the cell
             auto settle = [&](auto PHC, int s) __attribute__((always_inline)) {
                 constexpr int PH = decltype(PHC)::value;
                 // (a cell never passes lim; a NULL one grows by less than kPkDrift)
                 const uint32_t f = agree(q);
-                uint32_t M = pk_min(pk_add(Mr[PH][c], f), lim[c]);
+                const uint32_t before = Mr[PH][c];
+                uint32_t M = pk_min(pk_add(before, f), lim[c]);
                 const uint32_t more = f & FULL;
-                if (pk_any(more)) extend_more(M, lim[c], more, b, c);
+                uint32_t len = 0;
+                if constexpr (BT) len = pk_sub(M, before);
+                if (pk_any(more)) {
+                    extend_more(M, lim[c], more, b, c);
+                    if constexpr (BT) {  // lengths a record does not hold
+                        len = pk_minu(pk_sub(M, before), kPkLong * 0x10001u);
+#pragma unroll 1
+                        for (int half = 0; half < 2; ++half) {
+                            if (((len >> (16 * half)) & 0xffffu) < kPkLong || pk_get(before, half) < 0) continue;
+                            const uint32_t e = (pk_sub(M, before) >> (16 * half)) & 0xffffu;
+                            const int i = atomicAdd(X + L::LC, 1);
+                            if (i >= kPackedLongWords / 3) continue;
+                            longs[3 * i] = (uint32_t)s;
+                            longs[3 * i + 1] = (uint32_t)(k0 + OWN * NW * c + half);
+                            longs[3 * i + 2] = e;
+                        }
+                    }
+                }
                 Mr[PH][c] = M;
+                if constexpr (BT) {
+                    // uniform base and a 32-bit lane offset: no vector address arithmetic
+                    asm volatile("" : "+s"(rs));
+                    *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(rs) + (uint32_t)lane4) = pk_mad(len, 0x00100010u, flags);
+                    rs += NC * 64;
+                }
                 if (special) {
                     auto at = [&](int place) -> int { return (int16_t)((uint32_t)__builtin_amdgcn_readlane((int)M, place >> 1) >> (16 * (place & 1))); };
                     if ((em & (1u << c)) && at(ptp) >= t) ev = min(ev, 4 * s + kPkEvEnd);
@@ -511,6 +656,13 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
                 mi[c] = pk_max(M3, I);
                 md[c] = pk_max(M3, D);
                 Mr[PH][c] = M;
+                if constexpr (BT) {
+                    constexpr uint32_t one = 0x00010001u;
+                    flags = pk_minu(pk_sub(M, Xc), one);
+                    flags = pk_mad(pk_minu(pk_sub(M, D), one), 2 * one, flags);
+                    flags = pk_mad(pk_minu(pk_sub(mi[c], I), one), 4 * one, flags);
+                    flags = pk_mad(pk_minu(pk_sub(md[c], D), one), 8 * one, flags);
+                }
                 fetch(pk_minu(M, lim[c]), b, q);
             };
             using P0 = std::integral_constant<int, 0>;
@@ -569,6 +721,9 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
             }
             // every wave reaches these limits at the same score
             if (s0 >= s_bound) { r = TSU_EINTERNAL; break; }
+            if constexpr (BT) {
+                if (s0 + kPkStep >= a.step_cap) { r = TSU_ECIGAR; break; }
+            }
             if constexpr (PROBE) {
                 if (s0 >= a.probe_cap) { r = kProbeStopped; break; }
             }
@@ -644,7 +799,22 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
                 if (lane == 0) a.probe_out[pi] = far;
             }
         }
-        if (tid == 0)
+        if constexpr (BT) {
+            __syncthreads();  // every wave's records written
+            if (w == 0) {
+                int st = !lds_at_zero ? TSU_EINTERNAL : score < 0 ? score : 0;
+                int64_t out_off = 0;
+                int32_t out_n = 0;
+                if (st == 0)
+                    st = pk_walk<NC, OWN, HL>(rec, longs, min(__builtin_amdgcn_readfirstlane(X[L::LC]), kPackedLongWords / 3), kb,
+                                              s0, score, p, t, a, &out_off, &out_n);
+                if (lane == 0) {
+                    a.run_off[pi] = out_off;
+                    a.run_n[pi] = out_n;
+                    a.scores[pi] = st ? st : score * a.g;
+                }
+            }
+        } else if (tid == 0)
             a.scores[pi] = !lds_at_zero ? TSU_EINTERNAL : score < 0 ? score : score * a.g;
         __syncthreads();  // LDS reused by the next pair of this workgroup
     }

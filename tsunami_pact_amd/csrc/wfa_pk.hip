@@ -1,32 +1,26 @@
-// Instances of the packed kernel (scaled penalties 2/3/1): one wave of 1, 3,
+// Shapes of the packed kernel (scaled penalties 2/3/1): one wave of 1, 3,
 // 5 or 9 chunks of 128 diagonals (windows of 64-128, 256, 512 and 1024), or
 // 2-16 waves of 9 chunks (windows of 2048 to 16384); with expanded or packed
-// sequences; and the probe, one wave of 5 chunks.
+// sequences, scores only or with backtrace records; and the probe, one wave
+// of 5 chunks.
 #include "wfa_pk.h"
 
 namespace tsu {
 
-template <int NW, int C>
-static KernelFn pick_pk_shape(const Shape& sh) {
-    if (sh.probe) {
-        if constexpr (NW == 1 && C == 5) return sh.queue && !sh.expand ? wfa_pk_kernel<1, 5, false, true, true> : nullptr;
-        return nullptr;
-    }
-    if (sh.expand) return sh.queue ? wfa_pk_kernel<NW, C, true, true> : wfa_pk_kernel<NW, C, true, false>;
-    return sh.queue ? wfa_pk_kernel<NW, C, false, true> : wfa_pk_kernel<NW, C, false, false>;
-}
+KernelFn pick_pk_w1(const Shape& sh);
+KernelFn pick_pk_w2(const Shape& sh);
+KernelFn pick_pk_w4(const Shape& sh);
+KernelFn pick_pk_w8(const Shape& sh);
+KernelFn pick_pk_w16(const Shape& sh);
 
 KernelFn pick_pk(const Shape& sh) {
-    if (!sh.fixed_242 || sh.bt) return nullptr;
-    switch (100 * sh.nw + sh.reg_c) {
-    case 101: return pick_pk_shape<1, 1>(sh);
-    case 103: return pick_pk_shape<1, 3>(sh);
-    case 105: return pick_pk_shape<1, 5>(sh);
-    case 109: return pick_pk_shape<1, 9>(sh);
-    case 209: return pick_pk_shape<2, 9>(sh);
-    case 409: return pick_pk_shape<4, 9>(sh);
-    case 809: return pick_pk_shape<8, 9>(sh);
-    case 1609: return pick_pk_shape<16, 9>(sh);
+    if (!sh.fixed_242) return nullptr;
+    switch (sh.nw) {
+    case 1: return pick_pk_w1(sh);
+    case 2: return pick_pk_w2(sh);
+    case 4: return pick_pk_w4(sh);
+    case 8: return pick_pk_w8(sh);
+    case 16: return pick_pk_w16(sh);
     default: return nullptr;
     }
 }
