@@ -525,6 +525,10 @@ bool tsu_host::use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len,
     r.nw = 1;
     r.win = 64;
     while (r.win < W) r.win *= 2;
+    // a window of 64 diagonals fills half a chunk: the one-wave kernel with a
+    // diagonal per lane is faster there (218,540 x 125 bp at up to 6.4%: 0.253
+    // against 0.289 ms); it does not record
+    if (r.win == 64 && !r.bt) return false;
     if (r.win <= 1024) {
         r.reg_c = r.win <= 128 ? 1 : r.win == 256 ? 3 : r.win == 512 ? 5 : 9;
     } else {

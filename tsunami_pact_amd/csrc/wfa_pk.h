@@ -105,6 +105,10 @@ __device__ __forceinline__ uint32_t pk_add(uint32_t a, uint32_t b) {
 __device__ __forceinline__ uint32_t pk_sub(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, (pk_u16)(__builtin_bit_cast(pk_u16, a) - __builtin_bit_cast(pk_u16, b)));
 }
+// saturating a - b (signed)
+__device__ __forceinline__ uint32_t pk_sub_sat(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(pk_s16, a), __builtin_bit_cast(pk_s16, b)));
+}
 __device__ __forceinline__ uint32_t pk_mul(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, (pk_u16)(__builtin_bit_cast(pk_u16, a) * __builtin_bit_cast(pk_u16, b)));
 }
@@ -155,24 +159,6 @@ typedef __attribute__((address_space(3))) const uint16_t pk_lds_u16;
 typedef __attribute__((address_space(3))) const uint32_t pk_lds_u32;
 __device__ __forceinline__ uint32_t pk_ld16(uint32_t a) { return *reinterpret_cast<pk_lds_u16*>((uintptr_t)a); }
 __device__ __forceinline__ uint32_t pk_ld32(uint32_t a) { return *reinterpret_cast<pk_lds_u32*>((uintptr_t)a); }
-
-// Bases that pattern[v..] and text[h..] agree on, at most lim (>= 1), from
-// the packed words of the text at LDS byte tb and of the pattern at pb, 16
-// bases per round.
-__device__ __forceinline__ uint32_t pk_lcp(uint32_t pb, uint32_t tb, uint32_t v, uint32_t h, uint32_t lim) {
-    uint32_t ap = pb + ((v >> 4) << 2), at = tb + ((h >> 4) << 2);
-    uint32_t p0 = pk_ld32(ap), t0 = pk_ld32(at);
-    uint32_t n = 0;
-    for (;;) {
-        const uint32_t p1 = pk_ld32(ap + 4), t1 = pk_ld32(at + 4);
-        const uint32_t x = __builtin_amdgcn_alignbit(p1, p0, 2 * v) ^ __builtin_amdgcn_alignbit(t1, t0, 2 * h);
-        if (x) { n += (uint32_t)__builtin_ctz(x) >> 1; break; }
-        n += 16;
-        if (n >= lim) break;
-        p0 = p1; t0 = t1; ap += 4; at += 4;
-    }
-    return min(n, lim);
-}
 
 // LDS layout (bytes) of a launch: with H the text's expanded words, then the
 // pattern's; then the text's packed words, then the pattern's; then 32-bit
@@ -382,8 +368,10 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
         // past their ends the text holds 1 bits and the pattern 0 bits per
         // base, so a compare that starts at a bound seldom matches
         for (int i = tid; i < sw; i += NT) {
-            sS[sw + i] = i < pw ? a.words[pr.p_off + i] : 0u;
-            uint32_t wt = i < tw ? a.words[pr.t_off + i] : 0x55555555u;
+            uint32_t wp = 0u, wt = 0x55555555u;
+            if (i < pw) wp = a.words[pr.p_off + i];
+            if (i < tw) wt = a.words[pr.t_off + i];
+            sS[sw + i] = wp;
             if (i == tw - 1 && (t & 15)) wt = (wt & ~(~0u << (2 * (t & 15)))) | (0x55555555u << (2 * (t & 15)));
             sS[i] = wt;
         }
@@ -465,9 +453,42 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
         // not yet computed holds NULL.
         const int dlo = -p - kb, dhi = min(t - kb, OWN * NC - 1), d0 = -kb;
 
-        // score 0: M[0][0] = 0, extended (every lane computes it)
-        const int m0 = min(p, t);
-        const int ext0 = m0 > 0 ? (int)pk_lcp(pb, tb, 0, 0, (uint32_t)m0) : 0;
+        // Bases that pattern[v..] and text[h..] agree on, at most left: all lanes
+        // compare 16 bases each, 1,024 at a time.
+        const uint32_t lane4 = 4u * (uint32_t)lane;
+        auto lcp_wave = [&](int v, uint32_t h, int left) __attribute__((always_inline)) -> uint32_t {
+            uint32_t n = 0;
+            while (left > 0) {
+                const uint32_t o = min(lane4, (uint32_t)(left >> 4) << 2);  // lanes past the end repeat its word
+                const uint32_t ap = o + (pb + (uint32_t)((v >> 4) * 4)), at = o + (tb + ((h >> 4) << 2));
+                const uint32_t x = __builtin_amdgcn_alignbit(pk_ld32(ap + 4), pk_ld32(ap), 2u * (uint32_t)v) ^
+                                   __builtin_amdgcn_alignbit(pk_ld32(at + 4), pk_ld32(at), 2 * h);
+                const uint64_t diff = __builtin_amdgcn_ballot_w64(x != 0);
+                if (diff) {
+                    const int q = __builtin_ctzll(diff);
+                    return n + (uint32_t)min(left, 16 * q + (__builtin_ctz((uint32_t)__builtin_amdgcn_readlane((int)x, q)) >> 1));
+                }
+                n += (uint32_t)min(left, 1024);
+                h += 1024; v += 1024; left -= 1024;
+            }
+            return n;
+        };
+        // Past a full first compare, one cell at a time (most steps have one or
+        // two such cells, and an accurate read's runs are long).
+        auto extend_wave = [&](uint32_t& M, uint32_t limc, int kc, uint64_t mask, int half) __attribute__((always_inline)) {
+            const int sh = 16 * half;
+            while (mask) {
+                const int l = __builtin_ctzll(mask);
+                mask &= mask - 1;
+                const uint32_t h = ((uint32_t)__builtin_amdgcn_readlane((int)M, l) >> sh) & 0xffffu;
+                const int left = (int)((((uint32_t)__builtin_amdgcn_readlane((int)limc, l) >> sh) & 0xffffu) - h);
+                const uint32_t n = lcp_wave((int)h - (kc + 2 * l + half), h, left);
+                M += lane == l ? n << sh : 0u;
+            }
+        };
+
+        // score 0: M[0][0] = 0, extended
+        const int ext0 = (int)lcp_wave(0, 0, min(p, t));
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             const int k = k0 + OWN * NW * c;
@@ -521,36 +542,6 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
             }
         };
 
-        // Past a full first compare, one cell at a time: all lanes compare 16
-        // bases each, 1,024 from its position on (most steps have one or two
-        // such cells, and an accurate read's runs are long).
-        const uint32_t lane4 = 4u * (uint32_t)lane;
-        auto extend_wave = [&](uint32_t& M, uint32_t limc, int kc, uint64_t mask, int half) __attribute__((always_inline)) {
-            while (mask) {
-                const int l = __builtin_ctzll(mask);
-                mask &= mask - 1;
-                const int sh = 16 * half;
-                uint32_t h = ((uint32_t)__builtin_amdgcn_readlane((int)M, l) >> sh) & 0xffffu;
-                int left = (int)((((uint32_t)__builtin_amdgcn_readlane((int)limc, l) >> sh) & 0xffffu) - h);
-                int v = (int)h - (kc + 2 * l + half);
-                uint32_t n = 0;
-                while (left > 0) {
-                    const uint32_t o = min(lane4, (uint32_t)(left >> 4) << 2);  // lanes past the end repeat its word
-                    const uint32_t ap = o + (pb + (uint32_t)((v >> 4) * 4)), at = o + (tb + ((h >> 4) << 2));
-                    const uint32_t x = __builtin_amdgcn_alignbit(pk_ld32(ap + 4), pk_ld32(ap), 2u * (uint32_t)v) ^
-                                       __builtin_amdgcn_alignbit(pk_ld32(at + 4), pk_ld32(at), 2 * h);
-                    const uint64_t diff = __builtin_amdgcn_ballot_w64(x != 0);
-                    if (diff) {
-                        const int q = __builtin_ctzll(diff);
-                        n += (uint32_t)min(left, 16 * q + (__builtin_ctz((uint32_t)__builtin_amdgcn_readlane((int)x, q)) >> 1));
-                        break;
-                    }
-                    n += (uint32_t)min(left, 1024);
-                    h += 1024; v += 1024; left -= 1024;
-                }
-                M += lane == l ? n << sh : 0u;
-            }
-        };
         // Cells whose first compare matched to its end go on from there:
         // while there are many, all by further compares; then one by one.
         auto extend_more = [&](uint32_t& M, uint32_t limc, uint32_t more, uint32_t b, int c) __attribute__((always_inline)) {
@@ -590,6 +581,19 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
             uint32_t em = endm, el = lom, eh = him;  // opaque: scalar bit tests, no predicates kept
             asm volatile("" : "+s"(em), "+s"(el), "+s"(eh));
             const uint32_t special = (em | el | eh) & (1u << c);
+            // The cells looked at after every score, as a threshold per half that
+            // no other cell exceeds: the end cell at t, or a window edge at 0.
+            uint32_t watch = 0x7fff7fffu;
+            if (special) {
+                auto cell = [&](int place, int at_least) {
+                    const uint32_t sh = 16u * (uint32_t)(place & 1);
+                    const uint32_t v = (watch & ~(0xffffu << sh)) | (((uint32_t)(at_least - 1) & 0xffffu) << sh);
+                    watch = lane == place >> 1 ? v : watch;
+                };
+                if (em & (1u << c)) cell(ptp, t);
+                if (el & (1u << c)) cell(plo, 0);
+                if (eh & (1u << c)) cell(phi, 0);
+            }
             Words q;
             uint32_t flags = 0;  // BT: record bits 0-3 of the score in flight
             uint32_t* rs = nullptr;  // the chunk's records of the next score (uniform)
@@ -627,7 +631,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
                     *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(rs) + (uint32_t)lane4) = pk_mad(len, 0x00100010u, flags);
                     rs += NC * 64;
                 }
-                if (special) {
+                if (special && pk_any(pk_sub_sat(watch, M) & 0x80008000u)) {
                     auto at = [&](int place) -> int { return (int16_t)((uint32_t)__builtin_amdgcn_readlane((int)M, place >> 1) >> (16 * (place & 1))); };
                     if ((em & (1u << c)) && at(ptp) >= t) ev = min(ev, 4 * s + kPkEvEnd);
                     // a non-NULL cell at a window edge could extend the range beyond it

@@ -1,6 +1,6 @@
 // Single-wave register kernel instances (scaled penalties 2/3/1, i.e. 4/6/2),
-// windows of 64, 128, 256 and 512 diagonals, for sequences longer than the
-// packed kernel takes.
+// windows of 64 diagonals, and of 128, 256 and 512 for sequences longer than
+// the packed kernel takes.
 #include "wfa_reg.h"
 
 namespace tsu {
