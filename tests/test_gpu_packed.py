@@ -104,3 +104,29 @@ def test_extensions_longer_than_a_record_holds(aligner, oracle):
         p, q = seq(rng, n), seq(rng, 300)
         pairs += [(q + "A" + p + "C" + q, q + "T" + p + "G" + q), (p + q, p + "ACGTAC" + q), ("A" * n + q, "A" * (n + 3) + q)]
     check(aligner, oracle, pairs, 512)
+
+
+@pytest.mark.parametrize("pairs_n,window", [(300, 512), (300, 1024), (200, 2048), (100, 4096), (40, 8192), (2, 24576)])
+def test_waves_per_pair_follow_the_pair_count(aligner, oracle, pairs_n, window):
+    """Few pairs take more waves each (5 or 3 chunks a wave instead of 9), and
+    pairs wider than 16,384 diagonals the widest window: the same scores."""
+    rng = random.Random(window)
+    bound = {512: 512, 1024: 1024, 2048: 2048, 4096: 4096, 8192: 8192, 24576: 16383}[window]
+    if window == 24576:
+        pairs = [(seq(rng, 12_500), seq(rng, 12_000)) for _ in range(pairs_n)]
+    else:
+        base = [seq(rng, bound - 60) for _ in range(20)]
+        pairs = [(p, edited(rng, p, rng.randrange(1, window // 16))) for p in (rng.choice(base) for _ in range(pairs_n))]
+        pairs = [(p, t) for p, t in pairs if max(len(p), len(t)) <= bound]
+    want, _, _ = oracle.wfa_batch(pairs, 4, 6, 2)
+    aligner.set_tune_table([{"waves_per_pair": 1, "capacity": window, "bucket_bound": bound}])
+    try:
+        b = aligner.batch(pairs)
+        say(f"{len(pairs)} pairs in {window} diagonals, batched")
+        got, _ = aligner.align_batched(b)
+        assert (got == want).all(), np.nonzero(got != want)[0][:5]
+        say("the first eight")
+        got, _ = aligner.align_batched(aligner.batch(pairs[:8]))
+        assert (got == want[:8]).all()
+    finally:
+        aligner.set_tune_table([])

@@ -512,13 +512,22 @@ int tsu_host::reg_waves(const tsu_ctx* ctx, int32_t W) {
 // 0.573 ms packed and 1.83 expanded (3 waves per CU).
 constexpr int64_t kPkMinWaves = 12;
 
+// Waves of a launch of n pairs (at 9 chunks a wave) up to which it takes four
+// times (up to twice as many: twice) the waves per pair: a launch that leaves
+// SIMDs idle ends with its longest pair, which more waves shorten.  192 pairs
+// of 30-60 kbp, 20.9 -> 19.5 ms; 30,000 mixed pairs (whose last launches are
+// small) 70.0 -> 68.7 ms; lines at 512 and 1024 measured alike or slower.
+constexpr int64_t kPkFewWaves = 256;
+
 // Packed kernel (scaled penalties 2/3/1, sequences of at most 32000 bases):
 // the window for capacity W, its waves and chunks, and whether the sequences
 // are expanded in LDS.  The plain form's windows decide which pairs fit:
 // 64 * 2^j diagonals up to 1,024, then 4,096 on; the other forms (queue-fed),
 // which re-run a pair that overflows, take 2,048 first.
-bool tsu_host::use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh) {
-    if (!tsu_host::fixed_242(ctx) || W > 16 * 1024 || max_len > kPackedMaxLen) return false;
+bool tsu_host::use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh, int64_t n) {
+    // the widest window is for score launches fed from the queue
+    const int32_t widest = sh.queue && !sh.bt ? kPackedMaxWindow : 16 * 1024;
+    if (!tsu_host::fixed_242(ctx) || W > widest || max_len > kPackedMaxLen) return false;
     Shape r = sh;
     r.pk = true;
     r.reg_c = 9;
@@ -533,7 +542,19 @@ bool tsu_host::use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len,
         r.reg_c = r.win <= 128 ? 1 : r.win == 256 ? 3 : r.win == 512 ? 5 : 9;
     } else {
         if (!r.queue) r.win = std::max(r.win, 4096);
-        r.nw = r.win / 1024;
+        if (r.win > 16 * 1024) r.win = kPackedMaxWindow;
+        r.nw = std::min(16, r.win / 1024);
+        if (r.win == kPackedMaxWindow) r.reg_c = 14;
+    }
+    // few pairs: more waves for each, fewer chunks per wave
+    if (r.queue && r.win >= 512 && r.win <= 8192) {
+        if (n * r.nw <= kPkFewWaves && r.win >= 1024 && r.win <= 4096) {
+            r.nw *= 4;
+            r.reg_c = 3;
+        } else if (n * r.nw <= 2 * kPkFewWaves) {
+            r.nw *= 2;
+            r.reg_c = r.win == 512 ? 3 : 5;
+        }
     }
     KArgs a = base_args(ctx);
     a.seq_words = seq_words_for(ctx, max_len);
@@ -548,9 +569,9 @@ bool tsu_host::use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len,
 // kernel for sequences of at most 32000 bases; beyond, offsets in 32 bits:
 // one wave for up to 512 diagonals, 2-16 waves of 8 chunks for up to 8192
 // (and the two sequences fit in LDS).
-static void use_register_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh) {
+static void use_register_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh, int64_t n = INT64_MAX / 64) {
     if (max_len > tsu_host::max_seq_len(ctx)) return;  // the register kernels stage both sequences in LDS
-    if (tsu_host::use_packed_kernel(ctx, W, max_len, sh)) return;
+    if (tsu_host::use_packed_kernel(ctx, W, max_len, sh, n)) return;
     Shape r = sh;
     if (int c = tsu_host::reg_chunks(ctx, W)) {
         r.reg_c = c;
@@ -765,7 +786,7 @@ int32_t tsu_host::initial_capacity(const tsu_ctx* ctx, int32_t bound) {
     return std::max<int32_t>(W, 16);
 }
 
-Shape tsu_host::batched_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, int nw_hint) {
+Shape tsu_host::batched_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, int nw_hint, int64_t n) {
     if (ctx->two_piece) {  // the 2-piece kernels, fed from the queue
         Shape s2{1, max_len <= 32000, true, false, true};
         s2.two_piece = true;
@@ -777,7 +798,7 @@ Shape tsu_host::batched_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, in
     sh.fixed_242 = tsu_host::fixed_242(ctx);
     // a tuned hint above 1 asks for the LDS kernel with that many waves
     if (nw_hint <= 1) {
-        use_register_kernel(ctx, W, max_len, sh);
+        use_register_kernel(ctx, W, max_len, sh, n);
         if (sh.reg_c) return sh;
     }
     tsu_host::place_sequences(ctx, sh, max_len);
@@ -848,13 +869,23 @@ int32_t tsu_host::probe_capacity(const tsu_ctx* ctx, const tsu_pair& pr, int32_t
         for (c = 64; c < w; c *= 2) {}
     } else if (w <= 1024) {
         c = 1024;
-    } else if (w <= 16384 || need <= 1.25 * 16384) {
+    } else if (w <= 16384 || (std::max(pr.p_len, pr.t_len) > kPackedMaxLen && need <= 1.25 * 16384)) {
         for (c = 4096; c < std::min<int64_t>(w, 16384); c *= 2) {}
+    } else if (std::max(pr.p_len, pr.t_len) <= kPackedMaxLen && (w <= kPackedMaxWindow || need <= 1.25 * kPackedMaxWindow)) {
+        c = kPackedMaxWindow;
     } else {
         c = (w + 16383) / 16384 * 16384;
     }
     // (a launch clamps it to what its longest pair can use)
     return (int32_t)std::min<int64_t>(c, 1 << 26);
+}
+
+// The capacity a pair that overflowed W is re-run at: twice W, but the packed
+// kernel's widest window before going beyond it.
+int32_t tsu_host::next_capacity(const tsu_ctx* ctx, int32_t W, int32_t max_len) {
+    int64_t w = 2ll * W;
+    if (fixed_242(ctx) && max_len <= kPackedMaxLen && W < kPackedMaxWindow && w > kPackedMaxWindow) w = kPackedMaxWindow;
+    return (int32_t)std::min<int64_t>(w, capacity_max(ctx, max_len));
 }
 
 // The probe launch over `ids` (reordered longest first; d_order holds at
@@ -1045,7 +1076,7 @@ static int batched_core(tsu_ctx* ctx, tsu_batch* b, const std::vector<int32_t>& 
         HIPCHK(hipEventCreate(&rn->e0), "hipEventCreate");
         HIPCHK(hipEventCreate(&rn->e1), "hipEventCreate");
         bool launched = false;
-        const Shape sh = batched_shape(ctx, rn->W, rn->max_len, rn->nw_hint);
+        const Shape sh = batched_shape(ctx, rn->W, rn->max_len, rn->nw_hint, (int64_t)rn->ids.size());
         int r = launch_shape(ctx, io_of(b), sh, rn->W, rn->order, (int32_t)rn->ids.size(), rn->max_len, 0, nullptr,
                              rn->stream, rn->counter, rn->e0, rn->e1, rn->ring, &launched);
         if (r != TSU_OK) return r;
@@ -1096,7 +1127,7 @@ static int batched_core(tsu_ctx* ctx, tsu_batch* b, const std::vector<int32_t>& 
             if (rn->W >= tsu_host::capacity_max(ctx, rn->max_len)) return overflow_at(ctx, rn->W, rn->max_len);
             retried += (int)again.size();
             auto nx = std::make_unique<Run>();
-            nx->W = (int32_t)std::min<int64_t>(2ll * rn->W, tsu_host::capacity_max(ctx, rn->max_len));
+            nx->W = tsu_host::next_capacity(ctx, rn->W, rn->max_len);
             nx->max_len = rn->max_len;
             nx->nw_hint = 0;  // wider re-runs take the default shape of their capacity
             nx->order = rn->order;      // the finished launch's region and counter
@@ -1200,8 +1231,10 @@ extern "C" int tsu_align_batched_noalloc(tsu_ctx* ctx, const uint32_t* d_words, 
         int32_t* region = d_order + base[(size_t)bi];
         for (int attempt = 0; !todo.empty(); ++attempt) {
             W = std::min<int32_t>(W, tsu_host::capacity_max(ctx, max_len));
-            const Shape sh = batched_shape(ctx, W, max_len, attempt == 0 ? nw_hint : 0);
-            if (!sh.lds_ring) {
+            const Shape sh = batched_shape(ctx, W, max_len, attempt == 0 ? nw_hint : 0, (int64_t)todo.size());
+            // (beyond 16,384 diagonals with 4/6/2 too, though a window that
+            // needs no ring in device memory exists: a documented bound)
+            if (!sh.lds_ring || (sh.pk && sh.win > 16 * 1024)) {
                 for (int32_t i : todo) scores[i] = TSU_EKOVERFLOW;
                 no_room = todo[0];
                 break;
@@ -1228,7 +1261,7 @@ extern "C" int tsu_align_batched_noalloc(tsu_ctx* ctx, const uint32_t* d_words, 
             if (!again.empty()) {
                 if (W >= tsu_host::capacity_max(ctx, max_len)) return overflow_at(ctx, W, max_len);
                 retried += (int)again.size();
-                W = (int32_t)std::min<int64_t>(2ll * W, tsu_host::capacity_max(ctx, max_len));
+                W = tsu_host::next_capacity(ctx, W, max_len);
             }
             todo.swap(again);
         }
@@ -1412,9 +1445,9 @@ namespace {
 // of up to 16,000 bases (longer pairs of a narrow window go to the LDS kernel
 // where their scores are known, else to a window of two waves).
 constexpr int32_t kRecordOneWaveMaxLen = 16000;
-bool use_packed_recorder(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh) {
+bool use_packed_recorder(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh, int64_t n = INT64_MAX / 64) {
     Shape r = sh;
-    if (!tsu_host::use_packed_kernel(ctx, W, max_len, r) || (r.nw == 1 && max_len > kRecordOneWaveMaxLen)) return false;
+    if (!tsu_host::use_packed_kernel(ctx, W, max_len, r, n) || (r.nw == 1 && max_len > kRecordOneWaveMaxLen)) return false;
     sh = r;
     return true;
 }

@@ -236,7 +236,7 @@ int64_t plan_flight(tsu_server* s, Slot& sl, int32_t W_entry, int* status) {
     if (!sl.probing) {
         if (!lp.sh.lds_ring) ring = tsu::ring_bytes(lp.sh, lp.W, ctx->rm, ctx->ri) * lp.grid;
         for (int32_t W2 = lp.W; W2 < full;) {
-            W2 = (int32_t)std::min<int64_t>(2ll * W2, full);
+            W2 = tsu_host::next_capacity(ctx, W2, lp.max_len);
             const Shape sh2 = tsu_host::batched_shape(ctx, W2, lp.max_len, 0);
             if (sh2.lds_ring) continue;
             KArgs a2 = a;
@@ -452,7 +452,7 @@ void retire(tsu_server* s, Slot& sl) {
         LaunchPlan lp;
         lp.first = 0;
         lp.count = (int32_t)again.size();
-        lp.W = (int32_t)std::min<int64_t>(2ll * W, tsu_host::capacity_max(ctx, max_len));
+        lp.W = tsu_host::next_capacity(ctx, W, max_len);
         lp.max_len = max_len;
         lp.sh = tsu_host::batched_shape(ctx, lp.W, max_len, 0);
         KArgs a = tsu_host::base_args(ctx);

@@ -112,7 +112,7 @@ int32_t capacity_full(int32_t p, int32_t t);
 // keeps its five rings in LDS) the widest window whose rings fit the LDS.
 int32_t capacity_max(const tsu_ctx* ctx, int32_t max_len);
 // Persistent-launch shape for capacity W (ring in HBM when LDS is too small).
-Shape batched_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, int nw_hint);
+Shape batched_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, int nw_hint, int64_t n = INT64_MAX / 64);
 // Tuned waves per pair for a bucket (0 when the autotuner has not run).
 int tuned_waves(const tsu_ctx* ctx, int32_t bound);
 // Tuned initial capacity for a bucket (0 when none was tuned).
@@ -142,9 +142,12 @@ int reg2p_chunks(const tsu_ctx* ctx, int32_t W, int32_t max_len);
 // Longest sequence the packed kernel takes: its offsets, and one past the
 // last one of a text with its padding, are exact in 16 bits.
 constexpr int32_t kPackedMaxLen = 32000;
+// Its widest window (16 waves of 14 chunks), for score launches fed from the
+// queue.
+constexpr int32_t kPackedMaxWindow = 24576;
 // Packed kernel for capacity W and sequences up to max_len: fills in sh, or
 // returns false where it does not apply.
-bool use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh);
+bool use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh, int64_t n = INT64_MAX / 64);
 // Record words per workgroup and score steps of a packed launch that records
 // scores up to s.
 inline int32_t packed_steps(int64_t s) { return (int32_t)(s + 2 + tsu::kPackedStep); }
@@ -162,6 +165,8 @@ constexpr int32_t kProbeCap = 240;
 // latency).
 constexpr double kProbeMargin = 1.1;
 constexpr double kProbeMarginServed = 1.2;
+// The capacity pairs that overflowed W are re-run at.
+int32_t next_capacity(const tsu_ctx* ctx, int32_t W, int32_t max_len);
 int32_t probe_capacity(const tsu_ctx* ctx, const tsu_pair& pr, int32_t progress, double margin = kProbeMargin);
 // The probe's kernel: one wave, 512 diagonals.
 inline void probe_shape(int32_t max_len, Shape& sh) {

@@ -20,4 +20,12 @@ KernelFn pick_pk_shape(const Shape& sh) {
     return sh.queue ? wfa_pk_kernel<NW, C, false, true> : wfa_pk_kernel<NW, C, false, false>;
 }
 
+// Shapes that only queue-fed launches take.
+template <int NW, int C>
+KernelFn pick_pk_queue(const Shape& sh) {
+    if (!sh.queue || sh.probe) return nullptr;
+    if (sh.bt) return sh.expand ? wfa_pk_kernel<NW, C, true, true, false, true> : wfa_pk_kernel<NW, C, false, true, false, true>;
+    return sh.expand ? wfa_pk_kernel<NW, C, true, true> : wfa_pk_kernel<NW, C, false, true>;
+}
+
 }  // namespace tsu
