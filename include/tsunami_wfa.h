@@ -313,10 +313,10 @@ int tsu_cigars_stats(const tsu_cigars* c, int64_t* state_bytes, int32_t* record_
 /* Which kernels recorded the backtraces of the call that made c, as a mask
  * of TSU_KERNEL_* bits.  No reference counterpart (the reference computes no
  * CIGAR on the GPU); for callers and tests that check which path ran. */
-#define TSU_KERNEL_REG1    0x01u  /* one wave per pair, wavefronts in registers */
-#define TSU_KERNEL_ML4     0x02u  /* 16 chunks per wave, 4 waves per pair */
-#define TSU_KERNEL_ML8     0x04u  /* 16 chunks per wave, 8 waves per pair */
-#define TSU_KERNEL_ML16    0x08u  /* 16 chunks per wave, 16 waves per pair */
+#define TSU_KERNEL_REG1    0x01u  /* wavefronts in registers, windows of up to 1,024 diagonals */
+#define TSU_KERNEL_ML4     0x02u  /* several waves per pair, windows of up to 4,096 diagonals */
+#define TSU_KERNEL_ML8     0x04u  /* several waves per pair, windows of up to 8,192 diagonals */
+#define TSU_KERNEL_ML16    0x08u  /* several waves per pair, windows of up to 16,384 diagonals */
 #define TSU_KERNEL_LDS     0x10u  /* rings in LDS (or HBM), records for every score */
 #define TSU_KERNEL_LDS_CK  0x20u  /* rings in LDS (or HBM), ring checkpoints */
 #define TSU_KERNEL_2P      0x40u  /* gap-affine 2-piece kernel, records for every score */

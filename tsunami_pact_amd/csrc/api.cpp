@@ -1441,22 +1441,23 @@ static int copy_to_host(tsu_ctx* ctx, void* dst, const void* src, size_t bytes, 
 
 namespace {
 
-// The packed kernel as a recorder: with one wave per pair it takes sequences
-// of up to 16,000 bases (longer pairs of a narrow window go to the LDS kernel
-// where their scores are known, else to a window of two waves).
-constexpr int32_t kRecordOneWaveMaxLen = 16000;
+// The packed kernel as a recorder: windows of up to 1,024 diagonals take
+// sequences of up to 16,000 bases (longer pairs go to the LDS kernel where
+// their scores are known, else to the next window).
+constexpr int32_t kRecordNarrowMaxLen = 16000;
 bool use_packed_recorder(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh, int64_t n = INT64_MAX / 64) {
     Shape r = sh;
-    if (!tsu_host::use_packed_kernel(ctx, W, max_len, r, n) || (r.nw == 1 && max_len > kRecordOneWaveMaxLen)) return false;
+    if (!tsu_host::use_packed_kernel(ctx, W, max_len, r, n) || (r.win <= 1024 && max_len > kRecordNarrowMaxLen)) return false;
     sh = r;
     return true;
 }
 
 // Kernel family of a CIGAR launch at capacity W for a pair of length len:
-// the waves of the packed kernel, or 0 for the LDS kernel.
+// the packed kernel's window (those of up to 1,024 diagonals together), or 0
+// for the LDS kernel.
 int bt_family(const tsu_ctx* ctx, int32_t W, int32_t len) {
     Shape sh{1, true, true, true, true};
-    return use_packed_recorder(ctx, W, len, sh) ? sh.nw : 0;
+    return use_packed_recorder(ctx, W, len, sh) ? std::max(sh.win, 1024) : 0;
 }
 
 // Highest scaled score a pair of lengths (p, t) can have: min(p, t)
@@ -1485,6 +1486,27 @@ struct RecordPlan {
     int32_t W, max_len, step_cap, win;
     int64_t recs, per_wg;
     bool at_window;  // the step bound is the window's: a pair past it needs a wider one
+    // in flight: workgroups, state, queue order and counter, stream
+    int64_t grid = 0;
+    uint32_t* state = nullptr;
+    int64_t state_words = 0;
+    int32_t *d_ids = nullptr, *counter = nullptr;
+    hipStream_t stream = nullptr;
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    bool finished = false;
+};
+
+// Record launches in flight: on every return their streams are drained and
+// their events destroyed before the buffers they use are freed.
+struct RecordFlight {
+    std::vector<std::unique_ptr<RecordPlan>> plans;
+    ~RecordFlight() {
+        for (auto& p : plans) {
+            if (p->stream) (void)hipStreamSynchronize(p->stream);
+            if (p->e0) (void)hipEventDestroy(p->e0);
+            if (p->e1) (void)hipEventDestroy(p->e1);
+        }
+    }
 };
 
 // The LDS-kernel launch for pairs wider than every register window.
@@ -1542,8 +1564,10 @@ private:
     int settle_wide(const std::vector<int32_t>& ids);
     int launch_wide_async(WidePlan& wp, const std::vector<int32_t>& ids);
     int plan_records(std::vector<RecordPlan>& plans, int64_t& runs_need);
-    void plan_group(int32_t W, bool placed, std::vector<int32_t>& ids, std::vector<RecordPlan>& plans, int64_t& runs_need);
-    int settle_plan(const RecordPlan& pl);
+    void plan_group(int32_t W, bool placed, std::vector<int32_t>& ids, std::vector<RecordPlan>& plans, int64_t& runs_need,
+                    int64_t s_known = -1);
+    int start_plan(RecordPlan& pl, hipStream_t stream);
+    int settle_plan(const RecordPlan& pl, std::vector<int32_t>& wider);
     int record_pass();
     int wide_pass();
     int score_first_pass();
@@ -1570,6 +1594,7 @@ private:
     std::vector<uint8_t> done;
     std::vector<uint8_t> scored;   // scored by the probe: records from the score-first path
     std::vector<int32_t> wide;     // pairs that overflowed the widest register window
+    std::vector<int32_t> wide_now; // those of them in the launch beside the record launches
     std::vector<int32_t> order;    // pairs of the score-first path
     WideAsync wide_async;          // declared after the buffers its launch uses: synchronised first
 };
@@ -1649,7 +1674,9 @@ int CigarCall::grow_runs(int64_t more) {
     if (need > runs_cap) {
         DevBuf<uint32_t> grown;
         HIPCHK(grown.alloc((size_t)need), "hipMalloc (runs)");
-        if (used0) HIPCHK(hipMemcpy(grown.p, d_runs.p, (size_t)used0 * 4, hipMemcpyDeviceToDevice), "hipMemcpy D2D");
+        // (a reservation that found no room is counted but holds nothing)
+        const size_t held = (size_t)std::min<int64_t>((int64_t)used0, runs_cap);
+        if (held) HIPCHK(hipMemcpy(grown.p, d_runs.p, held * 4, hipMemcpyDeviceToDevice), "hipMemcpy D2D");
         std::swap(grown.p, d_runs.p);
         std::swap(grown.n, d_runs.n);
         runs_cap = need;
@@ -1824,7 +1851,7 @@ int CigarCall::plan_records(std::vector<RecordPlan>& plans, int64_t& runs_need) 
         for (Group& g : groups) {
             int32_t ml = 0;
             for (int32_t i : g.ids) ml = std::max(ml, std::max(b->pairs[(size_t)i].p_len, b->pairs[(size_t)i].t_len));
-            if (bt_family(ctx, std::min<int32_t>(g.W, capacity_full(ml, ml)), ml) == 16) {
+            if (bt_family(ctx, std::min<int32_t>(g.W, capacity_full(ml, ml)), ml) == 16 * 1024) {
                 merged.W = std::max(merged.W, g.W);
                 merged.ids.insert(merged.ids.end(), g.ids.begin(), g.ids.end());
             } else {
@@ -1835,6 +1862,20 @@ int CigarCall::plan_records(std::vector<RecordPlan>& plans, int64_t& runs_need) 
         groups.swap(rest);
     }
     for (Group& g : groups) plan_group(g.W, g.placed, g.ids, plans, runs_need);
+    // the pairs the probe finished, at their own scores (those the one-wave
+    // recorder does not take are left to the score-first path)
+    {
+        std::vector<int32_t> known;
+        int64_t s = 0;
+        for (int32_t i = 0; i < b->n; ++i) {
+            const tsu_pair& pr = b->pairs[(size_t)i];
+            if (!scored[(size_t)i] || std::max(pr.p_len, pr.t_len) > kRecordNarrowMaxLen) continue;
+            known.push_back(i);
+            s = std::max<int64_t>(s, scores[i] / ctx->g);
+        }
+        if (!known.empty())
+            plan_group(std::max<int32_t>(capacity_for_score(ctx, s), 16), false, known, plans, runs_need, s);
+    }
     // widest windows first, longest pairs first among equals
     std::stable_sort(plans.begin(), plans.end(), [](const RecordPlan& x, const RecordPlan& y) {
         return x.win != y.win ? x.win > y.win : x.max_len > y.max_len;
@@ -1843,9 +1884,10 @@ int CigarCall::plan_records(std::vector<RecordPlan>& plans, int64_t& runs_need) 
 }
 
 // The record launch of one group at first capacity W, when a register kernel
-// records it (placed: W is the probe's prediction).
+// records it (placed: W is the probe's prediction; s_known >= 0: no pair's
+// scaled score is higher).
 void CigarCall::plan_group(int32_t W, bool placed, std::vector<int32_t>& ids, std::vector<RecordPlan>& plans,
-                           int64_t& runs_need) {
+                           int64_t& runs_need, int64_t s_known) {
     int32_t max_len = 0;
     int64_t s_len = 0;
     for (int32_t i : ids) {
@@ -1857,8 +1899,8 @@ void CigarCall::plan_group(int32_t W, bool placed, std::vector<int32_t>& ids, st
     Shape sh{default_waves(W), max_len <= 32000, true, true, true};
     sh.fixed_242 = true;
     int32_t win = 0;  // the kernel's own window
-    if (max_len > kRecordOneWaveMaxLen && max_len <= tsu_host::kPackedMaxLen && W <= 1024) W = 2048;
-    if (use_packed_recorder(ctx, W, max_len, sh)) {
+    if (max_len > kRecordNarrowMaxLen && max_len <= tsu_host::kPackedMaxLen && W <= 1024) W = 2048;
+    if (use_packed_recorder(ctx, W, max_len, sh, (int64_t)ids.size())) {
         win = sh.win;
     } else if (placed && W > 16 * 1024) {
         // predicted beyond every register window: straight to the launch
@@ -1874,6 +1916,7 @@ void CigarCall::plan_group(int32_t W, bool placed, std::vector<int32_t>& ids, st
     }
     // a window holding every diagonal of the longest pair never overflows
     int64_t s_cap = win >= capacity_full(max_len, max_len) ? s_len : std::min(s_len, score_for_capacity(ctx, win));
+    if (s_known >= 0) s_cap = std::min(s_cap, s_known);
     if (s_cap < 0) return;
     KArgs a = base_args(ctx);
     a.W = W;
@@ -1896,90 +1939,185 @@ void CigarCall::plan_group(int32_t W, bool placed, std::vector<int32_t>& ids, st
     const int64_t recs = tsu_host::packed_records(sh, step_cap);
     const int64_t per_wg = recs * 4;
     // pairs of the widest window may also be walked by the launch for
-    // wider pairs, beside later launches: room for their whole bound
+    // wider pairs, beside later launches: room for their whole bound; others
+    // by a launch in twice the window
     for (int32_t i : ids) {
         const tsu_pair& pr = b->pairs[(size_t)i];
         const int64_t sb = score_bound(ctx, pr.p_len, pr.t_len);
-        runs_need += 2 * ((win >= 16 * 1024 ? sb : std::min<int64_t>(step_cap, sb)) / unit) + 2;
+        runs_need += 2 * ((win >= 16 * 1024 ? sb : std::min<int64_t>(2 * step_cap, sb)) / unit) + 2;
     }
     tsu_host::order_longest_first(ids, b->pairs.data());
-    plans.push_back(RecordPlan{std::move(ids), sh, a, W, max_len, step_cap, win, recs, per_wg,
-                               s_cap == s_win && s_win < s_len});
+    RecordPlan pl{std::move(ids), sh, a, W, max_len, step_cap, win, recs, per_wg, s_cap == s_win && s_win < s_len};
+    pl.grid = bt_grid(sh, a, (int64_t)pl.ids.size(), per_wg);
+    if (pl.grid <= 0) { ids = std::move(pl.ids); return; }
+    // (at least what one pair takes in twice as many diagonals, for the pairs
+    // that overflow: about twice the chunks for twice the scores)
+    pl.state_words = (recs * (win < 16 * 1024 ? std::max<int64_t>(pl.grid, 5) : pl.grid) + 63) / 64 * 64;
+    plans.push_back(std::move(pl));
 }
 
-int CigarCall::settle_plan(const RecordPlan& pl) {
+// The scores of a finished launch; wider: its pairs that overflowed the
+// window, for a launch in twice as many diagonals.
+int CigarCall::settle_plan(const RecordPlan& pl, std::vector<int32_t>& wider) {
     for (int32_t i : pl.ids) {
         const int32_t v = sc2[(size_t)i];
+        const bool over = v == TSU_EKOVERFLOW || (v == TSU_ECIGAR && pl.at_window);
         if (v >= 0) { scores[i] = v; done[(size_t)i] = 1; }
-        else if (pl.win >= 16 * 1024 && (v == TSU_EKOVERFLOW || (v == TSU_ECIGAR && pl.at_window)))
-            wide.push_back(i);
-        else if (v != TSU_EKOVERFLOW && v != TSU_ECIGAR)
+        else if (over && pl.win >= 16 * 1024) wide.push_back(i);
+        else if (over) wider.push_back(i);
+        else if (v != TSU_ECIGAR)  // its step bound was the budget's: score first
             return fail(ctx, v, "pair " + std::to_string(i) + ": " + tsu_strerror(v));
     }
     return TSU_OK;
 }
 
-// 1) The record pass.  The widest windows go first: their pairs that need
-// more are then known, and run on the second stream beside the other
-// launches.
+// Queues one record launch on `stream`.
+int CigarCall::start_plan(RecordPlan& pl, hipStream_t stream) {
+    pl.stream = stream;
+    if (!pl.e0) HIPCHK(hipEventCreate(&pl.e0), "hipEventCreate");
+    if (!pl.e1) HIPCHK(hipEventCreate(&pl.e1), "hipEventCreate");
+    HIPCHK(hipMemcpyAsync(pl.d_ids, pl.ids.data(), pl.ids.size() * sizeof(int32_t), hipMemcpyHostToDevice, stream), "hipMemcpyAsync (order)");
+    KArgs a = pl.a;
+    a.rec_g = pl.state; a.rec_cap = pl.recs;
+    a.step_cap = pl.step_cap;
+    a.runs = d_runs.p; a.runs_cap = std::max<int64_t>(runs_cap, 1); a.runs_used = d_used.p;
+    a.run_off = d_run_off.p; a.run_n = d_run_n.p;
+    DevBuf<uint8_t> none;  // the packed kernel has no ring
+    bool launched = false;
+    int r = launch_shape(ctx, io_of(b), pl.sh, pl.W, pl.d_ids, (int32_t)pl.ids.size(), pl.max_len, pl.grid, &a, stream, pl.counter,
+                         pl.e0, pl.e1, none, &launched);
+    if (r != TSU_OK) return r;
+    if (!launched) return fail(ctx, TSU_EINTERNAL, "empty record launch");
+    cg->state_bytes = std::max(cg->state_bytes, pl.per_wg * pl.grid);
+    ++cg->record_launches;
+    cg->kernels |= tsu_host::kernel_bit(pl.sh);
+    ++launches;
+    return TSU_OK;
+}
+
+// 1) The record pass.  Every launch whose state fits the budget beside the
+// others is queued at once, over two streams, widest window first: a
+// persistent launch keeps its CUs until its queue drains, and the next
+// launches' workgroups take what it leaves, so the tails overlap (one launch
+// after another, each was waited for).  A pair that overflows its window is
+// recorded in twice as many diagonals behind the launch that found it.  Once
+// the launches of the widest window are done, the pairs wider than that run
+// on a third stream.
 int CigarCall::record_pass() {
-    std::vector<RecordPlan> plans;
+    std::vector<RecordPlan> planned;
     int64_t runs_need = 0;
-    int r0 = plan_records(plans, runs_need);
-    if (r0 != TSU_OK) return r0;
-    if (plans.empty() && wide.empty()) return TSU_OK;
+    int r = plan_records(planned, runs_need);
+    if (r != TSU_OK) return r;
+    if (planned.empty() && wide.empty()) return TSU_OK;
     runs_cap = std::max<int64_t>(runs_need, 1);
     HIPCHK(d_runs.alloc((size_t)runs_cap), "hipMalloc (runs)");
-    size_t k = 0;
-    for (; k < plans.size() && plans[k].win >= 16 * 1024; ++k) {
-        int r = launch_bt(plans[k].sh, plans[k].a, plans[k].W, plans[k].ids, plans[k].max_len, plans[k].recs,
-                          plans[k].step_cap, plans[k].per_wg);
-        if (r != TSU_OK) return r;
+    DevBuf<int32_t> d_ids, d_counters;  // outlive the launches (declared before them)
+    HIPCHK(d_ids.alloc((size_t)std::max(b->n, 1)), "hipMalloc (order)");
+    HIPCHK(d_counters.alloc(std::max<size_t>(planned.size(), 1)), "hipMalloc (counters)");
+    // queued work (the probe's pairs, the counters) is done before other streams start
+    HIPCHK(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    RecordFlight fl;
+    size_t ids_at = 0;
+    for (size_t j = 0; j < planned.size(); ++j) {
+        auto p = std::make_unique<RecordPlan>(std::move(planned[j]));
+        p->d_ids = d_ids.p + ids_at;
+        p->counter = d_counters.p + j;
+        ids_at += p->ids.size();
+        fl.plans.push_back(std::move(p));
     }
-    if (k > 0) {
-        HIPCHK(hipMemcpy(sc2.data(), b->d_scores, (size_t)b->n * sizeof(int32_t), hipMemcpyDeviceToHost), "hipMemcpy D2H");
-        for (size_t j = 0; j < k; ++j) {
-            int r = settle_plan(plans[j]);
+    hipStream_t streams[2] = {ctx->stream, ctx->stream3};
+    bool wide_tried = false;
+    for (size_t first = 0; first < fl.plans.size();) {
+        // the launches that fit the budget together
+        size_t last = first;
+        int64_t words = 0;
+        while (last < fl.plans.size() && (last == first || 4 * (words + fl.plans[last]->state_words) <= budget))
+            words += fl.plans[last++]->state_words;
+        void* base = nullptr;
+        HIPCHK(bt_reserve(ctx, 0, (size_t)words * 4, &base), "hipMalloc (records)");
+        double load[2] = {0, 0};
+        uint32_t* at = static_cast<uint32_t*>(base);
+        for (size_t j = first; j < last; ++j) {
+            RecordPlan& p = *fl.plans[j];
+            p.state = at;
+            at += p.state_words;
+            const int k = load[1] < load[0] ? 1 : 0;
+            for (int32_t i : p.ids) load[k] += (double)b->pairs[(size_t)i].p_len * p.win;
+            r = start_plan(p, streams[k]);
             if (r != TSU_OK) return r;
         }
-    }
-    if (!wide.empty() && k < plans.size()) {
-        // the state of the launches after it is reserved before the wide
-        // launch starts: freeing a buffer to grow it waits for the whole
-        // device, so growing one later would stall them until it ends
-        size_t need = 0;
-        for (size_t j = k; j < plans.size(); ++j) {
-            const int64_t grid = bt_grid(plans[j].sh, plans[j].a, (int64_t)plans[j].ids.size(), plans[j].per_wg);
-            need = std::max(need, (size_t)(plans[j].recs * grid) * 4);
+        for (size_t open = last - first; open > 0;) {
+            bool progressed = false;
+            for (size_t j = first; j < last; ++j) {
+                RecordPlan& p = *fl.plans[j];
+                if (p.finished) continue;
+                const hipError_t q = hipEventQuery(p.e1);
+                if (q == hipErrorNotReady) continue;
+                if (q != hipSuccess) return hip_fail(ctx, q, "hipEventQuery");
+                progressed = true;
+                float ms = 0.f;
+                HIPCHK(hipEventElapsedTime(&ms, p.e0, p.e1), "hipEventElapsedTime");
+                kms_total += ms;
+                HIPCHK(hipMemcpyAsync(sc2.data(), b->d_scores, (size_t)b->n * sizeof(int32_t), hipMemcpyDeviceToHost,
+                                      ctx->stream_io), "hipMemcpyAsync D2H (scores)");
+                HIPCHK(hipStreamSynchronize(ctx->stream_io), "hipStreamSynchronize");
+                std::vector<int32_t> wider;
+                r = settle_plan(p, wider);
+                if (r != TSU_OK) return r;
+                // wider, on the same stream, in the state this launch leaves
+                std::vector<RecordPlan> next;
+                int64_t unused = 0;
+                if (!wider.empty()) plan_group(2 * p.win, false, wider, next, unused);
+                if (!next.empty()) {
+                    const int64_t room = p.state_words / next[0].recs;
+                    next[0].grid = std::min(next[0].grid, room);
+                }
+                if (!next.empty() && next[0].grid > 0) {
+                    auto n = std::make_unique<RecordPlan>(std::move(next[0]));
+                    n->d_ids = p.d_ids;
+                    n->counter = p.counter;
+                    n->state = p.state;
+                    n->state_words = p.state_words;
+                    std::swap(n->e0, p.e0);
+                    std::swap(n->e1, p.e1);
+                    const hipStream_t s = p.stream;
+                    fl.plans[j] = std::move(n);
+                    r = start_plan(*fl.plans[j], s);
+                    if (r != TSU_OK) return r;
+                } else {
+                    p.finished = true;  // (pairs left over are scored first)
+                    --open;
+                }
+            }
+            // pairs wider than every window, once no launch can add to them
+            bool all_wide = last == fl.plans.size();
+            for (const auto& p : fl.plans) all_wide = all_wide && (p->finished || p->win < 16 * 1024);
+            if (all_wide && !wide.empty() && !wide_tried) {
+                wide_tried = true;
+                WidePlan wp = plan_wide(wide);
+                if (wp.per_wg * (int64_t)wide.size() <= budget) {
+                    wide_now = wide;
+                    r = launch_wide_async(wp, wide_now);
+                    if (r != TSU_OK) return r;
+                }
+            }
+            if (!progressed) std::this_thread::sleep_for(std::chrono::microseconds(50));
         }
-        void* p = nullptr;
-        HIPCHK(bt_reserve(ctx, 0, need, &p), "hipMalloc (records)");
-        WidePlan wp = plan_wide(wide);
-        if (wp.per_wg * (int64_t)wide.size() <= budget) {
-            int r = launch_wide_async(wp, wide);
-            if (r != TSU_OK) return r;
-        }
+        first = last;
     }
-    for (size_t j = k; j < plans.size(); ++j) {
-        int r = launch_bt(plans[j].sh, plans[j].a, plans[j].W, plans[j].ids, plans[j].max_len, plans[j].recs,
-                          plans[j].step_cap, plans[j].per_wg);
-        if (r != TSU_OK) return r;
-    }
+    if (fl.plans.empty() && !wide.empty()) return TSU_OK;  // the wide pass runs them
     if (wide_async.launched) {
         HIPCHK(hipStreamSynchronize(ctx->stream2), "hipStreamSynchronize");
         float ms = 0.f;
         HIPCHK(hipEventElapsedTime(&ms, wide_async.e0, wide_async.e1), "hipEventElapsedTime");
         kms_total += ms;
-    }
-    HIPCHK(hipMemcpy(sc2.data(), b->d_scores, (size_t)b->n * sizeof(int32_t), hipMemcpyDeviceToHost), "hipMemcpy D2H");
-    for (size_t j = k; j < plans.size(); ++j) {
-        int r = settle_plan(plans[j]);
+        HIPCHK(hipMemcpy(sc2.data(), b->d_scores, (size_t)b->n * sizeof(int32_t), hipMemcpyDeviceToHost), "hipMemcpy D2H");
+        r = settle_wide(wide_now);
         if (r != TSU_OK) return r;
-    }
-    if (wide_async.launched) {
-        int r = settle_wide(wide);
-        if (r != TSU_OK) return r;
-        wide.clear();
+        std::vector<int32_t> rest;
+        for (int32_t i : wide)
+            if (std::find(wide_now.begin(), wide_now.end(), i) == wide_now.end()) rest.push_back(i);
+        wide.swap(rest);
     }
     return TSU_OK;
 }
@@ -2231,8 +2369,8 @@ extern "C" int tsu_cigars_stats(const tsu_cigars* c, int64_t* state_bytes, int32
 uint32_t tsu_host::kernel_bit(const Shape& sh) {
     if (sh.ck) return TSU_KERNEL_LDS_CK;
     if (sh.two_piece) return sh.reg_c ? TSU_KERNEL_2P_REG : TSU_KERNEL_2P;
-    if (sh.reg_c > 0 && sh.nw == 1) return TSU_KERNEL_REG1;
-    if (sh.pk) return sh.nw <= 4 ? TSU_KERNEL_ML4 : sh.nw == 8 ? TSU_KERNEL_ML8 : TSU_KERNEL_ML16;
+    if (sh.pk)
+        return sh.win <= 1024 ? TSU_KERNEL_REG1 : sh.win <= 4096 ? TSU_KERNEL_ML4 : sh.win <= 8192 ? TSU_KERNEL_ML8 : TSU_KERNEL_ML16;
     if (sh.reg_c > 0) return TSU_KERNEL_REG1;
     return TSU_KERNEL_LDS;
 }
