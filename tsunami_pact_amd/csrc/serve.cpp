@@ -227,7 +227,7 @@ int64_t plan_flight(tsu_server* s, Slot& sl, int32_t W_entry, int* status) {
         tsu_host::probe_shape(lp.max_len, lp.sh);
     } else {
         lp.W = W_entry > 0 ? std::min(W_entry, full) : W0;
-        lp.sh = tsu_host::batched_shape(ctx, lp.W, lp.max_len, W_entry > 0 ? 0 : waves);
+        lp.sh = tsu_host::batched_shape(ctx, lp.W, lp.max_len, W_entry > 0 ? 0 : waves, sl.n);
     }
     a.W = lp.W;
     lp.grid = std::min<int64_t>(tsu_host::resident_grid(ctx, lp.sh, a, status), lp.count);
@@ -454,7 +454,7 @@ void retire(tsu_server* s, Slot& sl) {
         lp.count = (int32_t)again.size();
         lp.W = tsu_host::next_capacity(ctx, W, max_len);
         lp.max_len = max_len;
-        lp.sh = tsu_host::batched_shape(ctx, lp.W, max_len, 0);
+        lp.sh = tsu_host::batched_shape(ctx, lp.W, max_len, 0, lp.count);
         KArgs a = tsu_host::base_args(ctx);
         a.W = lp.W;
         a.seq_words = tsu_host::seq_words_for(ctx, max_len);
