@@ -565,6 +565,57 @@ bool tsu_host::use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len,
     return true;
 }
 
+// Waves per CU below which the packed kernel for any penalties keeps its
+// sequences packed: 20,000 x 1,000 bp at up to 5%, 5/6/2, 1.29 ms with lines
+// of 12 and 20, 1.19 with 24 and 32; 4,000 x 700 bp 0.297 ms up to 24, 0.318
+// with 32.
+constexpr int kPkgMinWaves = 24;
+
+// Packed kernel for any penalties (wfa_pkg.h), scores only, in place of the
+// ring or 2-piece register kernel of shape sh: with that kernel's window, and
+// where it fits in LDS too (so which launches fit, and which capacities a
+// form accepts, stay that kernel's).  Not with an opening of 0: a gap's
+// source would be the M of the same score.
+//   One gap piece: always (the ring kernel is 1.05 times slower at 64 bp and
+// 16 diagonals, 3.1 at 20,000 x 1,000 bp / 397, 5.6 at 1,200 bp / 957).
+//   Two: in place of the ring kernel always (1,900 diagonals, 23.7 -> 2.9
+// ms).  The register kernel keeps one pair per wave, so it is better where
+// many pairs are in flight, and the packed one with few pairs or 1,024
+// diagonals (755 diagonals: 200 pairs 0.46 -> 0.21 ms, 2,000 0.74 -> 0.62,
+// 4,000 1.15 -> 1.11, 50,000 11.0 -> 11.9; 666: 4,000 0.88 -> 0.90; 954:
+// 4,000 2.81 -> 1.40); up to 256 diagonals it is as fast (200 x 400 bp) or
+// slower (10,000: 0.21 -> 0.30).
+//   Waves: 9 or 10 chunks 0.85 ms with 4 waves, 1.08 with 8, 2.5 with 16; 5
+// chunks 0.52 with 2, 0.56 with 4; 2 chunks 0.159 with 2, 0.178 with 1.  Two
+// pieces have fewer pairs per CU, and take more: 7 chunks 1.11 ms with 8, 1.20
+// with 4.  Up to a pair per CU, a chunk each.
+static bool use_packed_any(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh, int64_t n) {
+    if (tsu_host::fixed_242(ctx) || sh.bt || max_len > tsu_host::kPackedMaxLen) return false;
+    if (ctx->os < 1 || (ctx->two_piece && ctx->o2s < 1)) return false;
+    if (sh.reg_c && (sh.reg_c < 8 || (sh.reg_c < 16 && n > 8 * ctx->cu_count))) return false;
+    // with two pieces the widest capacity may be narrower than a pair needs,
+    // and the packed kernel reports such a pair a score early
+    if (ctx->two_piece && sh.queue && W < capacity_full(max_len, max_len) && W >= tsu_host::capacity_max(ctx, max_len)) return false;
+    KArgs a = base_args(ctx);
+    a.W = W;
+    a.seq_words = seq_words_for(ctx, max_len);
+    if (tsu::lds_bytes(sh, a) > ctx->max_lds) return false;
+    Shape r = sh;
+    r.pk = true;
+    r.win = sh.reg_c ? 64 * sh.reg_c : W;
+    r.reg_e = sh.reg_c ? sh.reg_e : 0;
+    const int chunks = tsu::pkg_chunks(r.win);
+    r.nw = chunks > 1 ? 2 : 1;
+    const bool few = n <= ctx->cu_count;
+    while (r.nw < 16 && (few ? r.nw < chunks : ctx->two_piece ? 3 * r.nw < 2 * chunks : 5 * r.nw < 2 * chunks)) r.nw *= 2;
+    r.reg_c = (chunks + r.nw - 1) / r.nw;
+    r.expand = true;
+    r.expand = ctx->max_lds / tsu::lds_bytes(r, a) * r.nw >= kPkgMinWaves;
+    if (tsu::lds_bytes(r, a) > ctx->max_lds) return false;
+    sh = r;
+    return true;
+}
+
 // Register kernels when the penalties and the capacity allow: the packed
 // kernel for sequences of at most 32000 bases; beyond, offsets in 32 bits:
 // one wave for up to 512 diagonals, 2-16 waves of 8 chunks for up to 8192
@@ -572,6 +623,7 @@ bool tsu_host::use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len,
 static void use_register_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh, int64_t n = INT64_MAX / 64) {
     if (max_len > tsu_host::max_seq_len(ctx)) return;  // the register kernels stage both sequences in LDS
     if (tsu_host::use_packed_kernel(ctx, W, max_len, sh, n)) return;
+    if (use_packed_any(ctx, W, max_len, sh, n)) return;
     Shape r = sh;
     if (int c = tsu_host::reg_chunks(ctx, W)) {
         r.reg_c = c;
@@ -588,7 +640,7 @@ static void use_register_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, 
     if (tsu::lds_bytes(r, a) <= ctx->max_lds) sh = r;
 }
 
-static Shape plain_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, bool* fits) {
+static Shape plain_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, int32_t n, bool* fits) {
     if (ctx->two_piece) {
         Shape s2{1, max_len <= 32000, true, false, false};
         s2.two_piece = true;
@@ -598,11 +650,12 @@ static Shape plain_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, bool* f
         a.W = W;
         a.seq_words = seq_words_for(ctx, max_len);
         *fits = tsu::lds_bytes(s2, a) <= ctx->max_lds;
+        if (*fits) use_packed_any(ctx, W, max_len, s2, n);
         return s2;
     }
     Shape sh{default_waves(W), max_len <= 32000, true, false, false};
     sh.fixed_242 = tsu_host::fixed_242(ctx);
-    use_register_kernel(ctx, W, max_len, sh);
+    use_register_kernel(ctx, W, max_len, sh, n);
     tsu_host::place_sequences(ctx, sh, max_len);
     KArgs a = base_args(ctx);
     a.W = W;
@@ -635,7 +688,7 @@ extern "C" int tsu_align_plain(tsu_ctx* ctx, tsu_batch* b, int32_t wf_length, in
     HIPCHK(hipSetDevice(ctx->device), "hipSetDevice");
     const double w0 = now_ms();
     bool fits = false;
-    Shape sh = plain_shape(ctx, W, b->max_len, &fits);
+    Shape sh = plain_shape(ctx, W, b->max_len, b->n, &fits);
     if (sh.two_piece && !fits)
         return fail(ctx, TSU_EINVAL, "tsu_align_plain: 2-piece rings for wf_length " + std::to_string(W) + " do not fit in LDS");
     if (!fits) {
@@ -668,18 +721,22 @@ extern "C" int tsu_align_plain(tsu_ctx* ctx, tsu_batch* b, int32_t wf_length, in
     }
     int launches = 1;
     const bool clean = lowest >= 0;
-    if (!clean && sh.two_piece && sh.reg_c) {
+    if (!clean && (sh.two_piece ? sh.reg_c > 0 : sh.pk && !sh.fixed_242)) {
         // the 2-piece register kernel stops past its score limit with an
-        // overflow status: such pairs get the LDS-ring kernel at the same
-        // capacity, so whether a pair fits depends on the capacity and not on
-        // that limit (the re-run's launch counts in the wall time)
-        const double r0 = now_ms();
-        std::vector<int32_t> again;
-        for (int32_t i = 0; i < b->n; ++i)
-            if (scores[i] == TSU_EKOVERFLOW) again.push_back(i);
-        if (!again.empty()) {
-            Shape s2{1, b->max_len <= 32000, true, false, true};
-            s2.two_piece = true;
+        // overflow status, and the packed kernel for any penalties when a
+        // cell comes to the window's edge: such pairs get the ring kernel at
+        // the same capacity, so whether a pair fits depends on the capacity
+        // and on neither (the re-run's launch counts in the wall time)
+        Shape s2{sh.two_piece ? 1 : default_waves(W), b->max_len <= 32000, true, false, true};
+        s2.two_piece = sh.two_piece;
+        s2.reg_e = sh.reg_e;
+        if (sh.pk) s2.reg_c = tsu_host::reg2p_chunks(ctx, W, b->max_len);
+        for (;;) {
+            const double r0 = now_ms();
+            std::vector<int32_t> again;
+            for (int32_t i = 0; i < b->n; ++i)
+                if (scores[i] == TSU_EKOVERFLOW) again.push_back(i);
+            if (again.empty()) break;
             DevBuf<int32_t> d_order;
             HIPCHK(d_order.alloc(again.size()), "hipMalloc (order)");
             HIPCHK(hipMemcpy(d_order.p, again.data(), again.size() * sizeof(int32_t), hipMemcpyHostToDevice), "hipMemcpy (order)");
@@ -693,6 +750,8 @@ extern "C" int tsu_align_plain(tsu_ctx* ctx, tsu_batch* b, int32_t wf_length, in
             r = copy_to_host(ctx, scores, b->d_scores, (size_t)b->n * sizeof(int32_t));
             if (r != TSU_OK) return r;
             d2h += now_ms() - d0;
+            if (s2.reg_c == 0) break;
+            s2.reg_c = 0;
         }
     }
     if (t) {
@@ -792,6 +851,7 @@ Shape tsu_host::batched_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, in
         s2.two_piece = true;
         s2.reg_c = tsu_host::reg2p_chunks(ctx, W, max_len);
         s2.reg_e = 10 * ctx->es + ctx->e2s;
+        use_packed_any(ctx, W, max_len, s2, n);
         return s2;
     }
     Shape sh{nw_hint > 0 ? nw_hint : default_waves(W), max_len <= 32000, true, false, true};
@@ -1310,12 +1370,12 @@ extern "C" int tsu_autotune(tsu_ctx* ctx, tsu_batch* b, int32_t sample_pairs) {
         // pairs per CU; pairs that overflow are re-run at the full one, and
         // that time is counted), and, where that capacity needs several
         // waves, capacity 0: each pair placed by the probe; otherwise the
-        // LDS kernel with 1-16 waves.
+        // automatic shape (1) and the LDS kernel with 2-16 waves.
         int32_t max_len = 0;
         for (int32_t i : sample) max_len = std::max(max_len, std::max(b->pairs[(size_t)i].p_len, b->pairs[(size_t)i].t_len));
         const int32_t W0 = initial_capacity(ctx, std::min(kBucketBounds[bi], max_len));
         std::vector<tsu_tune_entry> cands;
-        if (batched_shape(ctx, W0, max_len, 1).reg_c > 0) {
+        if (tsu_host::fixed_242(ctx) && batched_shape(ctx, W0, max_len, 1).reg_c > 0) {
             if (W0 > 1024) cands.push_back(tsu_tune_entry{1, 0, kBucketBounds[bi], 0});
             cands.push_back(tsu_tune_entry{1, W0, kBucketBounds[bi], 0});
             if (W0 / 2 >= 256) cands.push_back(tsu_tune_entry{1, W0 / 2, kBucketBounds[bi], 0});

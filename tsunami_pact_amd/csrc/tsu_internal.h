@@ -92,17 +92,23 @@ struct Shape {
     bool ck = false;         // backtrace from ring checkpoints (bt and queue set, LDS kernel)
     bool probe = false;      // single-wave register kernel stopping at KArgs::probe_cap
     bool gseq = false;       // LDS kernel reading the sequences from HBM (too long for LDS; int32 offsets)
-    bool pk = false;         // packed kernel: nw waves of reg_c chunks of 128 diagonals, two per register
+    bool pk = false;         // packed kernel (without fixed_242: for any penalties): nw waves of up to reg_c chunks of 128 diagonals, two per register
     bool expand = false;     // packed kernel with the sequences expanded in LDS
-    int win = 0;             // packed kernel: the window's width in diagonals (KArgs::W of the launch)
-    int reg_e = 0;           // 2-piece register kernel: 10 e1 + e2 after the gcd (11, 21 or 31)
+    int win = 0;             // packed kernels: the window's width in diagonals (KArgs::W of the launch)
+    int reg_e = 0;           // 2-piece register kernel (or the packed one in its place): 10 e1 + e2 after the gcd (11, 21 or 31)
 };
 
 // Packed kernel: scores it computes between two exchanges (it may record
 // that many scores past the end), and the words behind a workgroup's records
 // that list extensions too long for one (three words each).
 constexpr int kPackedStep = 6;
+// The 2-piece register kernel's last score: past it a pair overflows.
+constexpr int kP2RegMaxScore = 16000;
 constexpr int kPackedLongWords = 768;
+// Packed kernel for any penalties: own diagonals of a chunk, and the chunks
+// of a window.
+constexpr int kPkgOwn = 128 - 2 * kPackedStep;
+constexpr int pkg_chunks(int W) { return (W + kPkgOwn - 1) / kPkgOwn; }
 
 // Device scratch of tsu_align_batched_noalloc (a file-scope array per GPU):
 // work counters, then one queue-order entry per pair.

@@ -50,7 +50,6 @@
 namespace tsu {
 
 // doubled NULL-fed values (-32768 + 2 per score) stay negative this long
-constexpr int kP2RegMaxScore = 16000;
 
 constexpr int gcd_c(int a, int b) { return b ? gcd_c(b, a % b) : a; }
 

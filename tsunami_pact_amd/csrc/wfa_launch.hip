@@ -20,6 +20,8 @@ KernelFn pick_regmw(const Shape& sh);
 int regmw_exchange_words(int nw);
 KernelFn pick_pk(const Shape& sh);
 int64_t lds_bytes_pk(const Shape& sh, const KArgs& a);
+KernelFn pick_pkg(const Shape& sh);
+int64_t lds_bytes_pkg(const Shape& sh, const KArgs& a);
 KernelFn pick_2p(const Shape& sh);
 int64_t lds_bytes_2p(const Shape& sh, const KArgs& a);
 
@@ -41,8 +43,8 @@ int64_t ring_bytes(const Shape& sh, int32_t W, int32_t rm, int32_t ri) {
 }
 
 int64_t lds_bytes(const Shape& sh, const KArgs& a) {
+    if (sh.pk) return sh.fixed_242 ? lds_bytes_pk(sh, a) : lds_bytes_pkg(sh, a);
     if (sh.two_piece) return lds_bytes_2p(sh, a);
-    if (sh.pk) return lds_bytes_pk(sh, a);
     if (sh.reg_c > 0) {
         // sequences + misc (one wave), + the edge exchange area (several waves)
         const int ex = sh.nw == 1 ? 16 : regmw_exchange_words(sh.nw);
@@ -54,8 +56,8 @@ int64_t lds_bytes(const Shape& sh, const KArgs& a) {
 }
 
 static KernelFn pick(const Shape& sh) {
+    if (sh.pk) return sh.fixed_242 ? pick_pk(sh) : pick_pkg(sh);
     if (sh.two_piece) return pick_2p(sh);
-    if (sh.pk) return pick_pk(sh);
     if (sh.reg_c > 0) return sh.nw == 1 ? pick_reg(sh) : pick_regmw(sh);
     switch (sh.nw) {
     case 1: return pick_nw1(sh);
@@ -120,7 +122,10 @@ int occupancy(const Shape& sh, int64_t lds, int* blocks_per_cu) {
 
 int launch_wfa(const Shape& sh, const KArgs& args, int64_t grid, void* stream) {
     KArgs a = args;
-    if (sh.pk) a.W = sh.win;  // the packed kernel's windows are wider than the capacity asked for
+    if (sh.pk) {
+        a.W = sh.win;  // the packed kernel's windows are wider than the capacity asked for
+        if (!sh.fixed_242) a.probe_cap = sh.reg_e ? kP2RegMaxScore : 0x3fffffff;  // wfa_pkg.h
+    }
     KernelFn f = pick(sh);
     if (!f) return (int)hipErrorInvalidValue;
     if (grid <= 0) return 0;

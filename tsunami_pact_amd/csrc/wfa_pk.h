@@ -159,6 +159,8 @@ typedef __attribute__((address_space(3))) const uint16_t pk_lds_u16;
 typedef __attribute__((address_space(3))) const uint32_t pk_lds_u32;
 __device__ __forceinline__ uint32_t pk_ld16(uint32_t a) { return *reinterpret_cast<pk_lds_u16*>((uintptr_t)a); }
 __device__ __forceinline__ uint32_t pk_ld32(uint32_t a) { return *reinterpret_cast<pk_lds_u32*>((uintptr_t)a); }
+typedef __attribute__((address_space(3))) uint32_t pk_lds_w32;
+__device__ __forceinline__ void pk_st32(uint32_t a, uint32_t v) { *reinterpret_cast<pk_lds_w32*>((uintptr_t)a) = v; }
 
 // LDS layout (bytes) of a launch: with H the text's expanded words, then the
 // pattern's; then the text's packed words, then the pattern's; then 32-bit
@@ -171,6 +173,134 @@ __host__ __device__ constexpr uint32_t pk_expanded_entries(uint32_t seq_words) {
     return H ? 16 * seq_words + kPkPadBases - 24 : 0;
 }
 __host__ __device__ constexpr uint32_t pk_packed_words(uint32_t seq_words) { return seq_words + kPkPadBases / 16; }
+
+// Both sequences' packed words into LDS (text at sS, pattern sw words on).
+// Past their ends the text holds 1 bits and the pattern 0 bits per base, so a
+// compare that starts at a bound seldom matches.
+__device__ __forceinline__ void pk_stage(const uint32_t* words, const KPair& pr, int p, int t, uint32_t* sS, int sw, int tid, int nt) {
+    const int pw = (p + 15) >> 4, tw = (t + 15) >> 4;
+    for (int i = tid; i < sw; i += nt) {
+        uint32_t wp = 0u, wt = 0x55555555u;
+        if (i < pw) wp = words[pr.p_off + i];
+        if (i < tw) wt = words[pr.t_off + i];
+        sS[sw + i] = wp;
+        if (i == tw - 1 && (t & 15)) wt = (wt & ~(~0u << (2 * (t & 15)))) | (0x55555555u << (2 * (t & 15)));
+        sS[i] = wt;
+    }
+}
+// Their expanded words (hn positions each, the text's at x, the pattern's
+// after it): two positions per 32-bit word, from a window of 16 bases.
+__device__ __forceinline__ void pk_expand(uint32_t* x, uint32_t hn, const uint32_t* sS, int sw, int tid, int nt) {
+    for (int i = tid; i < (int)hn / 2; i += nt) {
+        const int j = i >> 3;
+        const uint32_t sh = 4u * (uint32_t)i;
+        const uint32_t wt = __builtin_amdgcn_alignbit(sS[j + 1], sS[j], sh);
+        const uint32_t wp = __builtin_amdgcn_alignbit(sS[sw + j + 1], sS[sw + j], sh);
+        x[i] = (wt & 0xffffu) | ((wt >> 2) << 16);
+        x[hn / 2 + i] = (wp & 0xffffu) | ((wp >> 2) << 16);
+    }
+}
+
+// Bases that pattern[v..] and text[h..] agree on, at most left, from the
+// packed words at LDS bytes pb and tb: all lanes of the wave compare 16 bases
+// each, 1,024 at a time.  Arguments and result are the same on every lane
+// (but lane4, four times the lane).
+__device__ __forceinline__ uint32_t pk_lcp_wave(uint32_t pb, uint32_t tb, uint32_t lane4, int v, uint32_t h, int left) {
+    uint32_t n = 0;
+    while (left > 0) {
+        const uint32_t o = min(lane4, (uint32_t)(left >> 4) << 2);  // lanes past the end repeat its word
+        const uint32_t ap = o + (pb + (uint32_t)((v >> 4) * 4)), at = o + (tb + ((h >> 4) << 2));
+        const uint32_t x = __builtin_amdgcn_alignbit(pk_ld32(ap + 4), pk_ld32(ap), 2u * (uint32_t)v) ^
+                           __builtin_amdgcn_alignbit(pk_ld32(at + 4), pk_ld32(at), 2 * h);
+        const uint64_t diff = __builtin_amdgcn_ballot_w64(x != 0);
+        if (diff) {
+            const int q = __builtin_ctzll(diff);
+            return n + (uint32_t)min(left, 16 * q + (__builtin_ctz((uint32_t)__builtin_amdgcn_readlane((int)x, q)) >> 1));
+        }
+        n += (uint32_t)min(left, 1024);
+        h += 1024; v += 1024; left -= 1024;
+    }
+    return n;
+}
+
+// The compares of two cells' extensions.
+template <bool H>
+struct PkCompare {
+    uint32_t tb, pb;  // LDS bytes of the packed text and pattern
+    static constexpr uint32_t FULL = H ? 0x00080008u : 0x00100010u;  // a half's compare matched to its end
+    // Reads and result apart, so that arithmetic fits between them.
+    struct Words {
+        uint32_t r[H ? 4 : 8];
+        uint32_t s[H ? 1 : 4];
+    };
+    // The compares from position cl (text) and cl - k (pattern); b: the
+    // lane's and chunk's part of the pattern's address for the high half.
+    __device__ __forceinline__ void fetch(uint32_t cl, uint32_t b, Words& q) const {
+        const uint32_t ha = pk_lo2(cl), hb = pk_hi2(cl);
+        const uint32_t va = ha + b, vb = hb + b;  // va is 2 short
+        if constexpr (H) {
+            q.r[0] = pk_ld16(ha);
+            q.r[1] = pk_ld16(va + 2);
+            q.r[2] = pk_ld16(hb);
+            q.r[3] = pk_ld16(vb);
+        } else {
+            const uint32_t va2 = va + 2;
+            // (the text's words start at LDS 0; an offset doubled is a bit position)
+            const uint32_t ap = (va2 >> 3) & ~3u, at = (ha >> 3) & ~3u, bp = (vb >> 3) & ~3u, bt = (hb >> 3) & ~3u;
+            q.r[0] = pk_ld32(at); q.r[1] = pk_ld32(at + 4);
+            q.r[2] = pk_ld32(ap); q.r[3] = pk_ld32(ap + 4);
+            q.r[4] = pk_ld32(bt); q.r[5] = pk_ld32(bt + 4);
+            q.r[6] = pk_ld32(bp); q.r[7] = pk_ld32(bp + 4);
+            q.s[0] = ha; q.s[1] = va2; q.s[2] = hb; q.s[3] = vb;
+        }
+    }
+    // Bases (at most 8 with H, 16 without) on which the sequences agree.
+    __device__ __forceinline__ uint32_t agree(const Words& q) const {
+        if constexpr (H) {
+            // bit 16 ends a full match
+            const uint32_t xa = pk_xad(q.r[0], q.r[1], 0x10000u), xb = pk_xad(q.r[2], q.r[3], 0x10000u);
+            return pk_half((uint32_t)__builtin_ctz(xa) | ((uint32_t)__builtin_ctz(xb) << 16));
+        } else {
+            const uint32_t xa = __builtin_amdgcn_alignbit(q.r[1], q.r[0], q.s[0]) ^ __builtin_amdgcn_alignbit(q.r[3], q.r[2], q.s[1]);
+            const uint32_t xb = __builtin_amdgcn_alignbit(q.r[5], q.r[4], q.s[2]) ^ __builtin_amdgcn_alignbit(q.r[7], q.r[6], q.s[3]);
+            // (all ones where nothing differs: 0xffff in that half)
+            const uint32_t fa = xa ? (uint32_t)__builtin_ctz(xa) : 0xffffffffu;
+            const uint32_t fb = xb ? (uint32_t)__builtin_ctz(xb) : 0xffffffffu;
+            return pk_minu(pk_half(__builtin_amdgcn_perm(fb, fa, 0x05040100u)), 0x00100010u);
+        }
+    }
+    // Past a full compare, one cell at a time by the whole wave (most steps
+    // have one or two such cells, and an accurate read's runs are long).
+    // kc: diagonal of the chunk's first lane.
+    __device__ __forceinline__ void extend_wave(uint32_t& M, uint32_t lim, int kc, int lane, uint64_t mask, int half) const {
+        const int sh = 16 * half;
+        while (mask) {
+            const int l = __builtin_ctzll(mask);
+            mask &= mask - 1;
+            const uint32_t h = ((uint32_t)__builtin_amdgcn_readlane((int)M, l) >> sh) & 0xffffu;
+            const int left = (int)((((uint32_t)__builtin_amdgcn_readlane((int)lim, l) >> sh) & 0xffffu) - h);
+            const uint32_t n = pk_lcp_wave(pb, tb, 4u * (uint32_t)lane, (int)h - (kc + 2 * l + half), h, left);
+            M += lane == l ? n << sh : 0u;
+        }
+    }
+    // Cells whose compare matched to its end go on from there: while there
+    // are many, all by further compares; then one by one.
+    __device__ __forceinline__ void extend_more(uint32_t& M, uint32_t lim, uint32_t more, uint32_t b, int kc, int lane) const {
+        uint64_t ml = __builtin_amdgcn_ballot_w64((more & 0xffffu) != 0), mh = __builtin_amdgcn_ballot_w64((more >> 16) != 0);
+        while (__builtin_popcountll(ml) + __builtin_popcountll(mh) > kPkWaveExtends) {
+            const uint32_t cl = pk_minu(M, lim);
+            Words q;
+            fetch(cl, b, q);
+            const uint32_t e = pk_minu(agree(q), pk_sub(lim, cl));
+            M = pk_add(M, e);
+            ml = __builtin_amdgcn_ballot_w64((e & FULL & 0xffffu) != 0);
+            mh = __builtin_amdgcn_ballot_w64((e & FULL) >> 16 != 0);
+        }
+        asm volatile("" : "+s"(kc));
+        extend_wave(M, lim, kc, lane, ml, 0);
+        extend_wave(M, lim, kc, lane, mh, 1);
+    }
+};
 
 template <int NW, int C>
 struct PkLayout {
@@ -364,30 +494,12 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
         const KPair pr = a.pairs[pi];
         const int p = __builtin_amdgcn_readfirstlane(pr.p_len);
         const int t = __builtin_amdgcn_readfirstlane(pr.t_len);
-        const int pw = (p + 15) >> 4, tw = (t + 15) >> 4;
-        // past their ends the text holds 1 bits and the pattern 0 bits per
-        // base, so a compare that starts at a bound seldom matches
-        for (int i = tid; i < sw; i += NT) {
-            uint32_t wp = 0u, wt = 0x55555555u;
-            if (i < pw) wp = a.words[pr.p_off + i];
-            if (i < tw) wt = a.words[pr.t_off + i];
-            sS[sw + i] = wp;
-            if (i == tw - 1 && (t & 15)) wt = (wt & ~(~0u << (2 * (t & 15)))) | (0x55555555u << (2 * (t & 15)));
-            sS[i] = wt;
-        }
+        pk_stage(a.words, pr, p, t, sS, sw, tid, NT);
         for (int i = L::XCH + tid; i < L::WORDS; i += NT)
             X[i] = i < L::PG ? (int32_t)kPkNull : i == L::EV ? kPkNoEvent : 0;
         __syncthreads();
         if constexpr (H) {
-            // two positions per 32-bit word: a window of 16 bases at 2i gives both
-            for (int i = tid; i < (int)hn / 2; i += NT) {
-                const int j = i >> 3;
-                const uint32_t sh = 4u * (uint32_t)i;
-                const uint32_t wt = __builtin_amdgcn_alignbit(sS[j + 1], sS[j], sh);
-                const uint32_t wp = __builtin_amdgcn_alignbit(sS[sw + j + 1], sS[sw + j], sh);
-                smem[i] = (wt & 0xffffu) | ((wt >> 2) << 16);
-                smem[hn / 2 + i] = (wp & 0xffffu) | ((wp >> 2) << 16);
-            }
+            pk_expand(smem, hn, sS, sw, tid, NT);
             __syncthreads();
         }
 
@@ -453,42 +565,11 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
         // not yet computed holds NULL.
         const int dlo = -p - kb, dhi = min(t - kb, OWN * NC - 1), d0 = -kb;
 
-        // Bases that pattern[v..] and text[h..] agree on, at most left: all lanes
-        // compare 16 bases each, 1,024 at a time.
         const uint32_t lane4 = 4u * (uint32_t)lane;
-        auto lcp_wave = [&](int v, uint32_t h, int left) __attribute__((always_inline)) -> uint32_t {
-            uint32_t n = 0;
-            while (left > 0) {
-                const uint32_t o = min(lane4, (uint32_t)(left >> 4) << 2);  // lanes past the end repeat its word
-                const uint32_t ap = o + (pb + (uint32_t)((v >> 4) * 4)), at = o + (tb + ((h >> 4) << 2));
-                const uint32_t x = __builtin_amdgcn_alignbit(pk_ld32(ap + 4), pk_ld32(ap), 2u * (uint32_t)v) ^
-                                   __builtin_amdgcn_alignbit(pk_ld32(at + 4), pk_ld32(at), 2 * h);
-                const uint64_t diff = __builtin_amdgcn_ballot_w64(x != 0);
-                if (diff) {
-                    const int q = __builtin_ctzll(diff);
-                    return n + (uint32_t)min(left, 16 * q + (__builtin_ctz((uint32_t)__builtin_amdgcn_readlane((int)x, q)) >> 1));
-                }
-                n += (uint32_t)min(left, 1024);
-                h += 1024; v += 1024; left -= 1024;
-            }
-            return n;
-        };
-        // Past a full first compare, one cell at a time (most steps have one or
-        // two such cells, and an accurate read's runs are long).
-        auto extend_wave = [&](uint32_t& M, uint32_t limc, int kc, uint64_t mask, int half) __attribute__((always_inline)) {
-            const int sh = 16 * half;
-            while (mask) {
-                const int l = __builtin_ctzll(mask);
-                mask &= mask - 1;
-                const uint32_t h = ((uint32_t)__builtin_amdgcn_readlane((int)M, l) >> sh) & 0xffffu;
-                const int left = (int)((((uint32_t)__builtin_amdgcn_readlane((int)limc, l) >> sh) & 0xffffu) - h);
-                const uint32_t n = lcp_wave((int)h - (kc + 2 * l + half), h, left);
-                M += lane == l ? n << sh : 0u;
-            }
-        };
+        const PkCompare<H> cmp{tb, pb};
 
         // score 0: M[0][0] = 0, extended
-        const int ext0 = (int)lcp_wave(0, 0, min(p, t));
+        const int ext0 = (int)pk_lcp_wave(pb, tb, lane4, 0, 0, min(p, t));
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             const int k = k0 + OWN * NW * c;
@@ -498,68 +579,6 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
         if constexpr (NW > 1) __syncthreads();
         int s0 = 0;           // scores finished
         int ev = kPkNoEvent;  // this wave's first event
-
-        // The two cells' first compare from position cl: the bases (at most 8
-        // with H, 16 without) from there on which the sequences agree.
-        // Reads and result apart, so that several chunks' reads are in
-        // flight together.
-        constexpr uint32_t FULL = H ? 0x00080008u : 0x00100010u;  // a half's compare matched to its end
-        struct Words {
-            uint32_t r[H ? 4 : 8];
-            uint32_t s[H ? 1 : 4];
-        };
-        auto fetch = [&](uint32_t cl, uint32_t b, Words& q) __attribute__((always_inline)) {
-            const uint32_t ha = pk_lo2(cl), hb = pk_hi2(cl);
-            const uint32_t va = ha + b, vb = hb + b;  // va is 2 short
-            if constexpr (H) {
-                q.r[0] = pk_ld16(ha);
-                q.r[1] = pk_ld16(va + 2);
-                q.r[2] = pk_ld16(hb);
-                q.r[3] = pk_ld16(vb);
-            } else {
-                const uint32_t va2 = va + 2;
-                // (the text's words start at LDS 0; an offset doubled is a bit position)
-                const uint32_t ap = (va2 >> 3) & ~3u, at = (ha >> 3) & ~3u, bp = (vb >> 3) & ~3u, bt = (hb >> 3) & ~3u;
-                q.r[0] = pk_ld32(at); q.r[1] = pk_ld32(at + 4);
-                q.r[2] = pk_ld32(ap); q.r[3] = pk_ld32(ap + 4);
-                q.r[4] = pk_ld32(bt); q.r[5] = pk_ld32(bt + 4);
-                q.r[6] = pk_ld32(bp); q.r[7] = pk_ld32(bp + 4);
-                q.s[0] = ha; q.s[1] = va2; q.s[2] = hb; q.s[3] = vb;
-            }
-        };
-        auto agree = [&](const Words& q) __attribute__((always_inline)) -> uint32_t {
-            if constexpr (H) {
-                // bit 16 ends a full match
-                const uint32_t xa = pk_xad(q.r[0], q.r[1], 0x10000u), xb2 = pk_xad(q.r[2], q.r[3], 0x10000u);
-                return pk_half((uint32_t)__builtin_ctz(xa) | ((uint32_t)__builtin_ctz(xb2) << 16));
-            } else {
-                const uint32_t xa = __builtin_amdgcn_alignbit(q.r[1], q.r[0], q.s[0]) ^ __builtin_amdgcn_alignbit(q.r[3], q.r[2], q.s[1]);
-                const uint32_t xb2 = __builtin_amdgcn_alignbit(q.r[5], q.r[4], q.s[2]) ^ __builtin_amdgcn_alignbit(q.r[7], q.r[6], q.s[3]);
-                // (all ones where nothing differs: 0xffff in that half)
-                const uint32_t fa = xa ? (uint32_t)__builtin_ctz(xa) : 0xffffffffu;
-                const uint32_t fb = xb2 ? (uint32_t)__builtin_ctz(xb2) : 0xffffffffu;
-                return pk_minu(pk_half(__builtin_amdgcn_perm(fb, fa, 0x05040100u)), 0x00100010u);
-            }
-        };
-
-        // Cells whose first compare matched to its end go on from there:
-        // while there are many, all by further compares; then one by one.
-        auto extend_more = [&](uint32_t& M, uint32_t limc, uint32_t more, uint32_t b, int c) __attribute__((always_inline)) {
-            uint64_t ml = __builtin_amdgcn_ballot_w64((more & 0xffffu) != 0), mh = __builtin_amdgcn_ballot_w64((more >> 16) != 0);
-            while (__builtin_popcountll(ml) + __builtin_popcountll(mh) > kPkWaveExtends) {
-                const uint32_t cl = pk_minu(M, limc);
-                Words q;
-                fetch(cl, b, q);
-                const uint32_t e = pk_minu(agree(q), pk_sub(limc, cl));
-                M = pk_add(M, e);
-                ml = __builtin_amdgcn_ballot_w64((e & FULL & 0xffffu) != 0);
-                mh = __builtin_amdgcn_ballot_w64((e & FULL) >> 16 != 0);
-            }
-            int kc = kb - HALO + OWN * (NW * c + w);
-            asm volatile("" : "+s"(kc));
-            extend_wave(M, limc, kc, ml, 0);
-            extend_wave(M, limc, kc, mh, 1);
-        };
 
         // The next kPkStep scores of the chunk in slot CC.
         auto advance = [&](auto CC) __attribute__((always_inline)) {
@@ -594,7 +613,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
                 if (el & (1u << c)) cell(plo, 0);
                 if (eh & (1u << c)) cell(phi, 0);
             }
-            Words q;
+            typename PkCompare<H>::Words q;
             uint32_t flags = 0;  // BT: record bits 0-3 of the score in flight
             uint32_t* rs = nullptr;  // the chunk's records of the next score (uniform)
             if constexpr (BT) rs = rec + ((int64_t)(s0 + 1) * NC + NW * c + w) * 64;
@@ -602,14 +621,14 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
             auto settle = [&](auto PHC, int s) __attribute__((always_inline)) {
                 constexpr int PH = decltype(PHC)::value;
                 // (a cell never passes lim; a NULL one grows by less than kPkDrift)
-                const uint32_t f = agree(q);
+                const uint32_t f = cmp.agree(q);
                 const uint32_t before = Mr[PH][c];
                 uint32_t M = pk_min(pk_add(before, f), lim[c]);
-                const uint32_t more = f & FULL;
+                const uint32_t more = f & PkCompare<H>::FULL;
                 uint32_t len = 0;
                 if constexpr (BT) len = pk_sub(M, before);
                 if (pk_any(more)) {
-                    extend_more(M, lim[c], more, b, c);
+                    cmp.extend_more(M, lim[c], more, b, kb - HALO + OWN * (NW * c + w), lane);
                     if constexpr (BT) {  // lengths a record does not hold
                         len = pk_minu(pk_sub(M, before), kPkLong * 0x10001u);
 #pragma unroll 1
@@ -667,7 +686,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
                     flags = pk_mad(pk_minu(pk_sub(mi[c], I), one), 4 * one, flags);
                     flags = pk_mad(pk_minu(pk_sub(md[c], D), one), 8 * one, flags);
                 }
-                fetch(pk_minu(M, lim[c]), b, q);
+                cmp.fetch(pk_minu(M, lim[c]), b, q);
             };
             using P0 = std::integral_constant<int, 0>;
             using P1 = std::integral_constant<int, 1>;
