@@ -14,7 +14,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 PENS = [(1, 1, 1), (2, 3, 1), (5, 6, 2), (4, 2, 7), (7, 11, 3), (12, 1, 1), (1, 14, 1), (10, 3, 9), (3, 0, 1), (20, 40, 15),
-        (4, 6, 2, 24, 1), (5, 1, 3, 10, 1), (4, 5, 3, 20, 2), (2, 1, 9, 8, 4), (9, 3, 1, 1, 7), (3, 0, 2, 9, 1), (4, 4, 8, 40, 3)]
+        (4, 6, 2, 24, 1), (4, 6, 2, 12, 2), (5, 1, 3, 10, 1), (4, 5, 3, 20, 2), (2, 1, 9, 8, 4), (9, 3, 1, 1, 7), (3, 0, 2, 9, 1), (4, 4, 8, 40, 3)]
 
 
 def say(msg):

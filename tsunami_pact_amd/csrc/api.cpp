@@ -579,20 +579,21 @@ constexpr int kPkgMinWaves = 24;
 //   One gap piece: always (the ring kernel is 1.05 times slower at 64 bp and
 // 16 diagonals, 3.1 at 20,000 x 1,000 bp / 397, 5.6 at 1,200 bp / 957).
 //   Two: in place of the ring kernel always (1,900 diagonals, 23.7 -> 2.9
-// ms).  The register kernel keeps one pair per wave, so it is better where
-// many pairs are in flight, and the packed one with few pairs or 1,024
-// diagonals (755 diagonals: 200 pairs 0.46 -> 0.21 ms, 2,000 0.74 -> 0.62,
-// 4,000 1.15 -> 1.11, 50,000 11.0 -> 11.9; 666: 4,000 0.88 -> 0.90; 954:
-// 4,000 2.81 -> 1.40); up to 256 diagonals it is as fast (200 x 400 bp) or
-// slower (10,000: 0.21 -> 0.30).
+// ms).  In place of the register kernel, which runs a pair on one wave, with
+// 768 and 1,024 diagonals (755: 200 pairs 0.46 -> 0.20 ms, 4,000 1.15 ->
+// 0.74, 50,000 at 5% 21.8 -> 13.1; 954: 4,000 2.81 -> 1.41), and with 512 up
+// to eight pairs per CU (394: 200 pairs 0.156 -> 0.107, 2,000 0.239 -> 0.200,
+// 4,000 0.324 -> 0.302, 10,000 0.649 -> 0.649); up to 256 diagonals it is as
+// fast (200 x 400 bp) or slower (10,000: 0.21 -> 0.30).
 //   Waves: 9 or 10 chunks 0.85 ms with 4 waves, 1.08 with 8, 2.5 with 16; 5
 // chunks 0.52 with 2, 0.56 with 4; 2 chunks 0.159 with 2, 0.178 with 1.  Two
-// pieces have fewer pairs per CU, and take more: 7 chunks 1.11 ms with 8, 1.20
-// with 4.  Up to a pair per CU, a chunk each.
+// pieces have fewer pairs per CU, and take more: 7 chunks 19.2 ms with 8, 22.3
+// with 4 (and 13.1 with 8 and GI, GD in registers: wfa_pkg.h).  Up to a pair
+// per CU, a chunk each.
 static bool use_packed_any(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh, int64_t n) {
     if (tsu_host::fixed_242(ctx) || sh.bt || max_len > tsu_host::kPackedMaxLen) return false;
     if (ctx->os < 1 || (ctx->two_piece && ctx->o2s < 1)) return false;
-    if (sh.reg_c && (sh.reg_c < 8 || (sh.reg_c < 16 && n > 8 * ctx->cu_count))) return false;
+    if (sh.reg_c && (sh.reg_c < 8 || (sh.reg_c == 8 && n > 8 * ctx->cu_count))) return false;
     // with two pieces the widest capacity may be narrower than a pair needs,
     // and the packed kernel reports such a pair a score early
     if (ctx->two_piece && sh.queue && W < capacity_full(max_len, max_len) && W >= tsu_host::capacity_max(ctx, max_len)) return false;

@@ -31,8 +31,7 @@
 // What bounds it: instruction issue and LDS reads per chunk and score (45
 // vector, 20 scalar and 11 LDS instructions; vector units 63% busy at 5/6/2)
 // with one gap piece; with two, whose ring is two to four times as large, the
-// pairs that fit a CU (4/6/2/24/1 in 768 diagonals: 54 KB, two pairs; vector
-// units 32% busy).  Copying slot by slot at the exchange took 3.0 ms where
+// pairs that fit a CU (vector units 32% busy with two pairs, 4/6/2/24/1).  Copying slot by slot at the exchange took 3.0 ms where
 // copying ten slots per LDS instruction takes 2.2 (20,000 x 1,000 bp at 5%,
 // 5/6/2, 397 diagonals; now 2.07; the ring kernel 9.2).
 #pragma once
@@ -50,17 +49,30 @@ __host__ __device__ constexpr int pkg_m_slots(int x, int o, int o2) {
     const int a = x > o ? x : o;
     return a > o2 ? a : o2;
 }
-inline int64_t pkg_ring_bytes(const KArgs& a, bool two_piece, int W) {
-    const int64_t slots = pkg_m_slots(a.x, a.o, two_piece ? a.o2 : 0) + 2ll * a.e + (two_piece ? 2ll * a.e2 : 0);
-    return slots * pkg_chunks(W) * 256;
+// The 2-piece kernel with GI and GD in registers: the register kernel's
+// extensions and windows, a wave per chunk.
+inline bool pkg_in_registers(const Shape& sh) { return sh.two_piece && sh.reg_e && sh.nw == 8 && pkg_chunks(sh.win) <= 8; }
+inline int64_t pkg_ring_bytes(const Shape& sh, const KArgs& a) {
+    const int64_t m = pkg_m_slots(a.x, a.o, sh.two_piece ? a.o2 : 0), gi = 2ll * a.e + (sh.two_piece ? 2ll * a.e2 : 0);
+    return pkg_chunks(sh.win) * (m * 256 + gi * (pkg_in_registers(sh) ? 8 * kPkgHl : 256));
 }
 
-template <int NW, int P, bool H, bool QUEUE>
+// E1, E2 > 0 (two pieces; extensions of 1-3 after the gcd): GI and GD in
+// registers, a chunk per wave (NW >= chunks), their slots fixed by unrolling
+// the scores of a block; the edges' words go through LDS.  4/6/2/24/1 in 768
+// diagonals: 49 KB and three pairs per CU instead of 59 KB and two, six LDS
+// instructions a score less; 50,000 x 1,000 bp at 5% 19.2 -> 13.1 ms.
+// (Loading the M a score reads during the score before: 13.0, not kept, since
+// M must then be two scores old.)
+template <int NW, int P, bool H, bool QUEUE, int E1 = 0, int E2 = 0>
 __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
     static_assert(P == 1 || P == 2, "gap pieces");
+    constexpr bool RG = E1 > 0;
+    static_assert(!RG || (P == 2 && kPkStep % E1 == 0 && kPkStep % E2 == 0), "slots fixed within a block");
+    constexpr int EN1 = RG ? E1 : 1, EN2 = RG ? E2 : 1;
     constexpr int NT = NW * 64;
     constexpr int OWN = kPkgOwn, HL = kPkgHl;
-    constexpr int XI = 64 / (2 * HL), XR = ((2 * P + 1) * kPkStep + XI - 1) / XI;  // slots copied per round, rounds
+    constexpr int XI = 64 / (2 * HL), XR = ((RG ? 1 : 2 * P + 1) * kPkStep + XI - 1) / XI;  // slots copied per round, rounds
     extern __shared__ __align__(16) uint32_t smem[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -79,7 +91,8 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
     const uint32_t stride = (uint32_t)NC * 256u;           // bytes per slot
     const int R = pkg_m_slots(a.x, a.o, P == 2 ? a.o2 : 0);
     const int gi1 = R, gd1 = gi1 + a.e, gi2 = gd1 + a.e, gd2 = P == 2 ? gi2 + a.e2 : gi2;
-    const int slots = P == 2 ? gd2 + a.e2 : gi2;
+    const int slots = RG ? R : P == 2 ? gd2 + a.e2 : gi2;
+    const uint32_t gx = rb + (uint32_t)R * stride;         // RG: the G words exchanged (2 HL per register and chunk)
     const int ahead = max(R, P == 2 ? max(a.e, a.e2) : a.e);
     const uint32_t lane4 = 4u * (uint32_t)lane;
 
@@ -101,6 +114,9 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
         const int t = __builtin_amdgcn_readfirstlane(pr.t_len);
         pk_stage(a.words, pr, p, t, sS, sw, tid, NT);
         for (int i = tid; i < slots * NC * 64; i += NT) ring[i] = kPkNull;
+        if constexpr (RG) {
+            for (int i = tid; i < 2 * (E1 + E2) * NC * 2 * HL; i += NT) pk_st32(gx + 4u * (uint32_t)i, kPkNull);
+        }
         if (tid == 0) X[1] = kPkNoEvent;
         __syncthreads();
         if constexpr (H) {
@@ -143,7 +159,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
         const int col = lane % (2 * HL);
         const int own_lane = col < HL ? col : 64 - 2 * HL + col;      // the copy's lane
         const uint32_t from_lane = (uint32_t)(col < HL ? 64 - 2 * HL + col : col) * 4u;
-        const int cM = min(R, kPkStep), c1 = min(a.e, kPkStep), c2 = P == 2 ? min(a.e2, kPkStep) : 0;
+        const int cM = min(R, kPkStep), c1 = RG ? 0 : min(a.e, kPkStep), c2 = P == 2 && !RG ? min(a.e2, kPkStep) : 0;
         const int items = cM + 2 * c1 + 2 * c2;
         uint32_t xat[XR], xsize[XR], xstep[XR], xbase[XR];  // position in the ring; its size, step and place
 #pragma unroll
@@ -170,6 +186,11 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
         int g1 = 0, h1 = kPkStep + ahead - a.o, g2 = 0, h2 = P == 2 ? kPkStep + ahead - a.o2 : 0;  // diagonals each piece reaches
         auto reach = [](int& g, int& h, int e) __attribute__((always_inline)) { while (h >= e) { ++g; h -= e; } };
         const PkCompare<H> cmp{tb, pb};
+        // RG: slots of GI1, GD1, GI2 and GD2 in turn
+        uint32_t G[2 * EN1 + 2 * EN2];
+#pragma unroll
+        for (uint32_t& v : G) v = kPkNull;
+        const bool g_in = lane < HL || lane >= 64 - HL, g_out = (lane >= HL && lane < 2 * HL) || (lane >= 64 - 2 * HL && lane < 64 - HL);
         int s0 = 0, r = 0;
         const bool same = p == t && ext0 == t;
         while (!same) {
@@ -205,6 +226,22 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
                     for (int u = 0; u < XR; ++u)
                         if (u * XI < items && xbase[u] != kPkgNone) pk_st32(xbase[u] + xat[u] + (uint32_t)j * 256u + 4u * (uint32_t)own_lane, v[u]);
                 }
+                if constexpr (RG) {
+                    if (w >= jlo && w <= jhi && g_in) {
+                        const int from = lane < HL ? w - 1 : w + 1;
+                        const bool there = from >= 0 && from < NC;
+                        const uint32_t at = gx + 4u * (uint32_t)(from * 2 * HL + (lane < HL ? HL + lane : lane - (64 - HL)));
+#pragma unroll
+                        for (int q = 0; q < 2 * (E1 + E2); ++q) {
+                            G[q] = kPkNull;
+                            if (there) G[q] = pk_ld32(at + (uint32_t)(q * NC * 2 * HL) * 4u);
+                        }
+                    }
+                    if (s0 % kPkgRenull == 0) {
+#pragma unroll
+                        for (uint32_t& v : G) v = pk_renull(v);
+                    }
+                }
                 if (s0 % kPkgRenull == 0) {
                     for (int j = w; j < NC; j += NW)
                         for (int q = 0; q < slots; ++q) {
@@ -236,27 +273,19 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
                 if (at_hi) cell(phi, 0);
                 const bool special = at_end || at_lo || at_hi;
                 uint32_t qm = bm, qx = bx, qo = bo, qo2 = bo2, qg = bg, qg2 = bg2;
-#pragma unroll 1
-                for (int s = s0 + 1; s <= s0 + kPkStep; ++s) {
-                    const uint32_t ai1 = A1 + qg, ad1 = ai1 + eb;
-                    const uint32_t i1 = pk_ld32(ai1), d1 = pk_ld32(ad1);
+                auto up = [&](uint32_t v) __attribute__((always_inline)) -> uint32_t {
+                    const uint32_t u = __builtin_amdgcn_update_dpp(0u, v, 0x138, 0xF, 0xF, true);
+                    return pk_add(__builtin_amdgcn_alignbit(v, u, 16), 0x00010001u);
+                };
+                auto down = [&](uint32_t v) __attribute__((always_inline)) -> uint32_t {
+                    const uint32_t u = __builtin_amdgcn_update_dpp(0u, v, 0x130, 0xF, 0xF, true);
+                    return __builtin_amdgcn_alignbit(u, v, 16);
+                };
+                // Score s from the G slots it reads; put() gets their new values.
+                auto score = [&](int s, uint32_t i1, uint32_t d1, uint32_t i2, uint32_t d2, auto put) __attribute__((always_inline)) {
                     const uint32_t mx = pk_ld32(A + qx), mo = pk_ld32(A + qo);
-                    uint32_t ai2 = 0, ad2 = 0, i2 = 0, d2 = 0, mo2 = 0;
-                    if constexpr (P == 2) {
-                        ai2 = A2 + qg2;
-                        ad2 = ai2 + eb2;
-                        i2 = pk_ld32(ai2);
-                        d2 = pk_ld32(ad2);
-                        mo2 = pk_ld32(A + qo2);
-                    }
-                    auto up = [&](uint32_t v) __attribute__((always_inline)) -> uint32_t {
-                        const uint32_t u = __builtin_amdgcn_update_dpp(0u, v, 0x138, 0xF, 0xF, true);
-                        return pk_add(__builtin_amdgcn_alignbit(v, u, 16), 0x00010001u);
-                    };
-                    auto down = [&](uint32_t v) __attribute__((always_inline)) -> uint32_t {
-                        const uint32_t u = __builtin_amdgcn_update_dpp(0u, v, 0x130, 0xF, 0xF, true);
-                        return __builtin_amdgcn_alignbit(u, v, 16);
-                    };
+                    uint32_t mo2 = 0;
+                    if constexpr (P == 2) mo2 = pk_ld32(A + qo2);
                     uint32_t I1 = up(i1), D1 = down(d1), I2 = 0, D2 = 0;
                     const uint32_t Xc = pk_add(mx, 0x00010001u);
                     uint32_t M = pk_max(pk_max(D1, Xc), I1);
@@ -280,12 +309,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
                     const uint32_t cl = pk_minu(M, lim);
                     typename PkCompare<H>::Words q;
                     cmp.fetch(cl, pl, q);
-                    pk_st32(ai1, pk_max(mo, I1));
-                    pk_st32(ad1, pk_max(mo, D1));
-                    if constexpr (P == 2) {
-                        pk_st32(ai2, pk_max(mo2, I2));
-                        pk_st32(ad2, pk_max(mo2, D2));
-                    }
+                    put(pk_max(mo, I1), pk_max(mo, D1), pk_max(mo2, I2), pk_max(mo2, D2));
                     const uint32_t f = cmp.agree(q);
                     M = pk_add(M, pk_minu(f, pk_sub(lim, cl)));  // (a NULL cell has nothing left)
                     const uint32_t more = f & PkCompare<H>::FULL;
@@ -297,8 +321,37 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
                         if (at_lo && at(raw, kPkStep) >= 0) ev = min(ev, 4 * s + kPkEvEdge);
                         if (at_hi && at(raw, phi) >= 0) ev = min(ev, 4 * s + kPkEvEdge);
                     }
-                    qm = next(qm, Rb); qx = next(qx, Rb); qo = next(qo, Rb); qg = next(qg, eb);
-                    if constexpr (P == 2) { qo2 = next(qo2, Rb); qg2 = next(qg2, eb2); }
+                    qm = next(qm, Rb); qx = next(qx, Rb); qo = next(qo, Rb);
+                    if constexpr (P == 2) qo2 = next(qo2, Rb);
+                };
+                if constexpr (RG) {
+#pragma unroll
+                    for (int i = 1; i <= kPkStep; ++i) {
+                        uint32_t &gi = G[i % E1], &gd = G[E1 + i % E1], &gi2r = G[2 * E1 + i % E2], &gd2r = G[2 * E1 + E2 + i % E2];
+                        score(s0 + i, gi, gd, gi2r, gd2r, [&](uint32_t ni, uint32_t nd, uint32_t ni2, uint32_t nd2) __attribute__((always_inline)) {
+                            gi = ni; gd = nd; gi2r = ni2; gd2r = nd2;
+                        });
+                    }
+                    if (g_out) {
+                        const uint32_t at = gx + 4u * (uint32_t)(j * 2 * HL + (lane < 32 ? lane - HL : lane - (64 - 2 * HL) + HL));
+#pragma unroll
+                        for (int q = 0; q < 2 * (E1 + E2); ++q) pk_st32(at + (uint32_t)(q * NC * 2 * HL) * 4u, G[q]);
+                    }
+                } else {
+#pragma unroll 1
+                    for (int s = s0 + 1; s <= s0 + kPkStep; ++s) {
+                        const uint32_t ai1 = A1 + qg, ad1 = ai1 + eb, ai2 = A2 + qg2, ad2 = ai2 + eb2;
+                        const uint32_t i1 = pk_ld32(ai1), d1 = pk_ld32(ad1);
+                        uint32_t i2 = 0, d2 = 0;
+                        if constexpr (P == 2) { i2 = pk_ld32(ai2); d2 = pk_ld32(ad2); }
+                        score(s, i1, d1, i2, d2, [&](uint32_t ni, uint32_t nd, uint32_t ni2, uint32_t nd2) __attribute__((always_inline)) {
+                            pk_st32(ai1, ni);
+                            pk_st32(ad1, nd);
+                            if constexpr (P == 2) { pk_st32(ai2, ni2); pk_st32(ad2, nd2); }
+                        });
+                        qg = next(qg, eb);
+                        if constexpr (P == 2) qg2 = next(qg2, eb2);
+                    }
                 }
             }
             if (ev != kPkNoEvent) atomicMin(X + 1, ev);
