@@ -14,10 +14,12 @@
 // are its own and kPkStep at each end are copies of its neighbours'.  A cell
 // depends on its neighbours one diagonal away one score before, so from exact
 // copies a chunk computes kPkStep scores of its own diagonals without a word
-// from another chunk; then the chunks exchange the copies through LDS.  That
-// costs 10% more cells, and takes away, per chunk and score, the exchange of
-// edge values and, per score, the wait of the waves of a pair for each other
-// (a pair of 16 waves that met at every score spent half its time waiting).
+// from another chunk; then the chunks exchange the copies, through LDS, or
+// within a lone wave from register to register (ds_bpermute, which needs no
+// LDS memory).  That costs 10% more cells, and takes away, per chunk and
+// score, the exchange of edge values and, per score, the wait of the waves of
+// a pair for each other (a pair of 16 waves that met at every score spent
+// half its time waiting).
 //
 // State per chunk, five VGPRs and one bound:
 //   Mr[3]  M of the scores s-1, s-2, s-3 (slot s mod 3; the loop over scores
@@ -54,7 +56,7 @@
 // position, so the address of a compare is the offset itself, doubled: 8
 // instructions for the two cells against 20 with funnel shifts of the packed
 // words, at 4.5 instead of 0.5 bytes of LDS per base of a pair.  The host
-// takes H where that leaves enough waves per CU (pk_seq_expanded).
+// takes H where that leaves enough waves per CU.
 //
 // What bounds it: vector issue.  A chunk and score takes about 30 vector
 // instructions for 128 cells, where the kernels it replaced took 29-35 for
@@ -64,7 +66,11 @@
 // ring, a wait per score) and after: 30,000 pairs of 100-20,000 bp at 1-15%,
 // batched, 158 -> 73 ms; 10,000 pairs of up to 2,000 bp in one plain launch
 // of 4 waves per pair 1.63 -> 0.63 ms; 250,000 x 1,000 bp at 5% (one wave, 5
-// chunks) 7.18 -> 6.36 ms; 10,000 x 10,240 bp at up to 1% 0.71 -> 0.57 ms.
+// chunks) 7.18 -> 6.29 ms; 10,000 x 10,240 bp at up to 1% 0.71 -> 0.57 ms.
+// Without LDS for a lone wave's copies, and with the expanded pattern's
+// padding left to the words behind it, a 1,000 bp pair takes 4.8 KB, and 32
+// instead of 20 waves share a CU (0.63 vector instructions per cycle before):
+// 6.29 -> 5.39 ms; the ragged 2,000 bp pairs 0.735 -> 0.684.
 //
 // Recurrences, bounds and end tests: wfa_gpu.cu:253-331,610-631.
 #pragma once
@@ -164,7 +170,7 @@ __device__ __forceinline__ void pk_st32(uint32_t a, uint32_t v) { *reinterpret_c
 
 // LDS layout (bytes) of a launch: with H the text's expanded words, then the
 // pattern's; then the text's packed words, then the pattern's; then 32-bit
-// words for the queue index and the exchange.  (A cell among the copies may
+// words for the queue index and the exchange of several waves.  (A cell among the copies may
 // hold an offset h < k, whose pattern position h - k is negative but not
 // below -t - kPkPadBases: the pattern follows a text at least that long.)
 template <bool H>
@@ -172,7 +178,21 @@ __host__ __device__ constexpr uint32_t pk_expanded_entries(uint32_t seq_words) {
     // positions 0 .. max_len + kPkPadBases, even (16 * seq_words >= max_len + 32)
     return H ? 16 * seq_words + kPkPadBases - 24 : 0;
 }
+// The pattern's are fewer: past max_len + 16 a compare reads the words behind
+// them, for lanes at a bound, which have nothing left to extend.
+template <bool H>
+__host__ __device__ constexpr uint32_t pk_expanded_pattern(uint32_t seq_words) { return H ? 16 * seq_words - 16 : 0; }
+// (as far as one may read behind them, p + 122 positions)
+constexpr int64_t pk_expanded_reach(uint32_t seq_words) { return 2 * (pk_expanded_entries<true>(seq_words) + 16ll * seq_words + kPkPadBases); }
 __host__ __device__ constexpr uint32_t pk_packed_words(uint32_t seq_words) { return seq_words + kPkPadBases / 16; }
+
+// LDS bytes of a launch with `state` bytes behind the sequences.
+inline int64_t pk_lds_bytes(const Shape& sh, uint32_t sw, int64_t state) {
+    const int64_t packed = 8ll * pk_packed_words(sw) + state;
+    if (!sh.expand) return packed;
+    const int64_t x = 2ll * (pk_expanded_entries<true>(sw) + pk_expanded_pattern<true>(sw)) + packed;
+    return x > pk_expanded_reach(sw) ? x : pk_expanded_reach(sw);
+}
 
 // Both sequences' packed words into LDS (text at sS, pattern sw words on).
 // Past their ends the text holds 1 bits and the pattern 0 bits per base, so a
@@ -188,16 +208,16 @@ __device__ __forceinline__ void pk_stage(const uint32_t* words, const KPair& pr,
         sS[i] = wt;
     }
 }
-// Their expanded words (hn positions each, the text's at x, the pattern's
-// after it): two positions per 32-bit word, from a window of 16 bases.
-__device__ __forceinline__ void pk_expand(uint32_t* x, uint32_t hn, const uint32_t* sS, int sw, int tid, int nt) {
+// Their expanded words (the text's hn positions at x, the pattern's hp after
+// them): two positions per 32-bit word, from a window of 16 bases.
+__device__ __forceinline__ void pk_expand(uint32_t* x, uint32_t hn, uint32_t hp, const uint32_t* sS, int sw, int tid, int nt) {
     for (int i = tid; i < (int)hn / 2; i += nt) {
         const int j = i >> 3;
         const uint32_t sh = 4u * (uint32_t)i;
         const uint32_t wt = __builtin_amdgcn_alignbit(sS[j + 1], sS[j], sh);
         const uint32_t wp = __builtin_amdgcn_alignbit(sS[sw + j + 1], sS[sw + j], sh);
         x[i] = (wt & 0xffffu) | ((wt >> 2) << 16);
-        x[hn / 2 + i] = (wp & 0xffffu) | ((wp >> 2) << 16);
+        if (i < (int)hp / 2) x[hn / 2 + i] = (wp & 0xffffu) | ((wp >> 2) << 16);
     }
 }
 
@@ -316,7 +336,7 @@ struct PkLayout {
     static constexpr int XP = 5 * XR;                 // words per parity
     static constexpr int XCH = 4;
     static constexpr int MISC = 0;                    // [4] queue index
-    static constexpr int PG = XCH + 2 * XP;           // [NW] exchanges each wave has finished
+    static constexpr int PG = XCH + (NW > 1 ? 2 * XP : 0);  // [NW] exchanges each wave has finished
     static constexpr int EV = PG + (NW > 1 ? NW : 0); // [1] first event, score * 4 + kind
     static constexpr int LC = EV + 1;                 // [1] long extensions recorded
     static constexpr int WORDS = EV + 4;
@@ -458,9 +478,10 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
     const int lane = tid & 63;
     const int w = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t hn = pk_expanded_entries<H>((uint32_t)a.seq_words);
+    const uint32_t hp = pk_expanded_pattern<H>((uint32_t)a.seq_words);
     const uint32_t hpb = 2 * hn;  // pattern's expanded words (the text's start at 0)
     const int sw = (int)pk_packed_words((uint32_t)a.seq_words);
-    const uint32_t tb = 4 * hn;                   // packed words: text,
+    const uint32_t tb = 2 * (hn + hp);            // packed words: text,
     const uint32_t pb = tb + 4u * (uint32_t)sw;   // pattern
     uint32_t* sS = smem + tb / 4;
     int32_t* X = reinterpret_cast<int32_t*>(sS + 2 * sw);
@@ -499,7 +520,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
             X[i] = i < L::PG ? (int32_t)kPkNull : i == L::EV ? kPkNoEvent : 0;
         __syncthreads();
         if constexpr (H) {
-            pk_expand(smem, hn, sS, sw, tid, NT);
+            pk_expand(smem, hn, hp, sS, sw, tid, NT);
             __syncthreads();
         }
 
@@ -546,10 +567,12 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
         const uint32_t pl = (H ? hpb : 8u * pb) - 2u * (uint32_t)k0 - 2u;
         // this lane's word of the exchange for slot 0: what it copies out
         // (own diagonals at the chunk's ends) or takes in (copies)
-        const bool out_lane = HALO > 0 && ((lane >= HL && lane < 2 * HL) || (lane >= 64 - 2 * HL && lane < 64 - HL));
+        const bool out_lane = HALO > 0 && NW > 1 && ((lane >= HL && lane < 2 * HL) || (lane >= 64 - 2 * HL && lane < 64 - HL));
         const bool in_lane = HALO > 0 && (lane < HL || lane >= 64 - HL);
         uint32_t xl = 0;
-        if constexpr (HALO > 0) {
+        if constexpr (HALO > 0 && NW == 1) {
+            xl = 4u * (uint32_t)(lane < 32 ? 64 - 2 * HL + lane : lane - (64 - 2 * HL));  // the copied cell's lane
+        } else if constexpr (HALO > 0) {
             int word;  // chunk j's own are at (j + 1) 2 HL
             if (lane < HL) word = w * 2 * HL + HL + lane;                    // the last of j - 1
             else if (lane >= 64 - HL) word = (w + 2) * 2 * HL + lane - (64 - HL);  // the first of j + 1
@@ -584,7 +607,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
         auto advance = [&](auto CC) __attribute__((always_inline)) {
             constexpr int c = decltype(CC)::value;
             const int u = s0 / kPkStep;
-            if constexpr (HALO > 0) {
+            if constexpr (HALO > 0 && NW > 1) {
                 if (s0 > 0 && in_lane) {
                     const uint32_t x = xl + 4u * (uint32_t)(((u & 1) ^ 1) * L::XP + 2 * HL * NW * c);
                     Mr[0][c] = pk_ld32(x);
@@ -705,7 +728,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
             score(P0{}, std::false_type{}, s0 + 6);
             if (done()) return;
             settle(P0{}, s0 + 6);
-            if constexpr (HALO > 0) {
+            if constexpr (HALO > 0 && NW > 1) {
                 if (out_lane) {
                     int32_t* x = X + (xl - xb) / 4u + (u & 1) * L::XP + 2 * HL * NW * c;
                     x[0] = (int32_t)Mr[0][c];
@@ -773,6 +796,27 @@ __global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
                 }
             }
             act = __builtin_amdgcn_readfirstlane(act);
+            // one wave: the copies from the neighbour chunks' registers
+            auto take = [&](auto CC) __attribute__((always_inline)) {
+                constexpr int c = decltype(CC)::value;
+                if constexpr (HALO > 0 && NW == 1 && c < C) {
+                    if (act & (1u << c)) {
+                        auto from = [&](uint32_t (&v)[C]) __attribute__((always_inline)) {
+                            const uint32_t lo = c > 0 ? v[c > 0 ? c - 1 : 0] : kPkNull, hi = c + 1 < C ? v[c + 1 < C ? c + 1 : 0] : kPkNull;
+                            const uint32_t x = (uint32_t)__builtin_amdgcn_ds_bpermute((int)xl, (int)(lane < 32 ? hi : lo));
+                            v[c] = in_lane ? x : v[c];
+                        };
+                        from(Mr[0]); from(Mr[1]); from(Mr[2]); from(mi); from(md);
+                    }
+                }
+            };
+            if (s0 > 0) {
+                take(std::integral_constant<int, 0>{}); take(std::integral_constant<int, 1>{});
+                take(std::integral_constant<int, 2>{}); take(std::integral_constant<int, 3>{});
+                take(std::integral_constant<int, 4>{}); take(std::integral_constant<int, 5>{});
+                take(std::integral_constant<int, 6>{}); take(std::integral_constant<int, 7>{});
+                take(std::integral_constant<int, 8>{});
+            }
             auto sweep = [&](auto CC) __attribute__((always_inline)) {
                 if constexpr (decltype(CC)::value < C) {
                     if (act & (1u << decltype(CC)::value)) advance(CC);

@@ -48,8 +48,7 @@ int64_t lds_bytes_pk(const Shape& sh, const KArgs& a) {
     case 1609: x = PkLayout<16, 9>::WORDS; break;
     default: x = PkLayout<16, 14>::WORDS; break;
     }
-    const int64_t hn = sh.expand ? pk_expanded_entries<true>(sw) : 0;
-    return 4 * hn + 8ll * pk_packed_words(sw) + 4 * x;
+    return pk_lds_bytes(sh, sw, 4 * x);
 }
 
 }  // namespace tsu

@@ -78,9 +78,10 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
     const int lane = tid & 63;
     const int w = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t hn = pk_expanded_entries<H>((uint32_t)a.seq_words);
+    const uint32_t hp = pk_expanded_pattern<H>((uint32_t)a.seq_words);
     const uint32_t hpb = 2 * hn;
     const int sw = (int)pk_packed_words((uint32_t)a.seq_words);
-    const uint32_t tb = 4 * hn, pb = tb + 4u * (uint32_t)sw;
+    const uint32_t tb = 2 * (hn + hp), pb = tb + 4u * (uint32_t)sw;
     uint32_t* sS = smem + tb / 4;
     int32_t* X = reinterpret_cast<int32_t*>(sS + 2 * sw);  // [0] queue index, [1] first event
     uint32_t* ring = reinterpret_cast<uint32_t*>(X + 4);
@@ -120,7 +121,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
         if (tid == 0) X[1] = kPkNoEvent;
         __syncthreads();
         if constexpr (H) {
-            pk_expand(smem, hn, sS, sw, tid, NT);
+            pk_expand(smem, hn, hp, sS, sw, tid, NT);
             __syncthreads();
         }
 

@@ -9,8 +9,7 @@ KernelFn pick_pkg(const Shape& sh) { return sh.two_piece ? pick_pkg2p(sh) : pick
 
 int64_t lds_bytes_pkg(const Shape& sh, const KArgs& a) {
     const uint32_t sw = (uint32_t)a.seq_words;
-    const int64_t hn = sh.expand ? pk_expanded_entries<true>(sw) : 0;
-    return 4 * hn + 8ll * pk_packed_words(sw) + 16 + pkg_ring_bytes(sh, a);
+    return pk_lds_bytes(sh, sw, 16 + pkg_ring_bytes(sh, a));
 }
 
 }  // namespace tsu
