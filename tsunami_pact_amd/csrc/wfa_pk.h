@@ -460,13 +460,19 @@ __device__ __forceinline__ int pk_walk(const uint32_t* rec, const uint32_t* long
     return bt_end(w, out_off, out_n);
 }
 
+// Registers for five waves per SIMD: the 9-chunk score kernels would take 99
+// (four waves), and 96 cost no spill; 30,000 pairs of 100-20,000 bp, batched,
+// 71.8 -> 70.1 ms.  Six (80) spills.  From eight waves on a pair's waves come
+// in multiples of two per SIMD.
+constexpr int pk_waves_per_simd(int nw, int c, bool h, bool bt) { return c == 9 && h && !bt && nw <= 4 ? 5 : 1; }
+
 // W is the window's width in diagonals as the host counts it (it may be less
 // than the chunks hold): the range a pair may use is
 // [kmin, kmin + W - 1], kmin = max(-W/2, -p-1), moved down where it would
 // pass t + 1; a non-NULL cell on its first or last diagonal (where that is
 // no bound of the alignment) ends the pair with TSU_EKOVERFLOW.
 template <int NW, int C, bool H, bool QUEUE, bool PROBE = false, bool BT = false>
-__global__ __launch_bounds__(NW * 64) void wfa_pk_kernel(KArgs a) {
+__global__ __launch_bounds__(NW * 64, pk_waves_per_simd(NW, C, H, BT)) void wfa_pk_kernel(KArgs a) {
     static_assert(NW >= 1 && NW <= 16 && C >= 1 && C <= 16, "at most 16 waves of 16 chunks");
     static_assert(!PROBE || NW == 1, "the probe runs on one wave");
     using L = PkLayout<NW, C>;
