@@ -179,6 +179,9 @@ static void bt_release(tsu_ctx* ctx) {
         ctx->bt_buf[i] = nullptr;
         ctx->bt_bytes[i] = 0;
     }
+    for (const auto& c : ctx->bt_more) (void)hipFree(c.first);
+    ctx->bt_more.clear();
+    ctx->bt_budget = 0;
 }
 
 // Backtrace state buffer i with at least `bytes`, grown (never shrunk) in
@@ -193,6 +196,72 @@ static hipError_t bt_reserve(tsu_ctx* ctx, int i, size_t bytes, void** p) {
         ctx->bt_bytes[i] = bytes;
     }
     *p = ctx->bt_buf[i];
+    return hipSuccess;
+}
+
+// Room for records of the given sizes, each in one piece, in the buffers the
+// context holds (buffer 0 and bt_more).  The first is as large as the first
+// call needs.  Getting and giving back tens of GB takes seconds (77 GB of
+// written memory: 8 s), so a call that needs more adds a second one with all
+// that is left of `most` (the budget), and only if that does not do either
+// does one buffer take their place.  The launches that used them have
+// completed.
+static hipError_t bt_place(tsu_ctx* ctx, const std::vector<size_t>& bytes, size_t most, std::vector<void*>& at) {
+    auto round = [](size_t n) { return (n + 255) & ~(size_t)255; };
+    std::vector<std::pair<uint8_t*, size_t>> room;  // what is left of each buffer
+    room.emplace_back(static_cast<uint8_t*>(ctx->bt_buf[0]), ctx->bt_bytes[0]);
+    size_t held = ctx->bt_bytes[0];
+    for (const auto& c : ctx->bt_more) {
+        room.emplace_back(static_cast<uint8_t*>(c.first), c.second);
+        held += c.second;
+    }
+    at.assign(bytes.size(), nullptr);
+    auto place = [&](size_t j) -> bool {
+        for (auto& c : room)
+            if (c.first && c.second >= round(bytes[j])) {
+                at[j] = c.first;
+                c.first += round(bytes[j]);
+                c.second -= round(bytes[j]);
+                return true;
+            }
+        return false;
+    };
+    size_t missing = 0, all = 0;
+    for (size_t j = 0; j < bytes.size(); ++j) {
+        all += round(bytes[j]);
+        if (!place(j)) missing += round(bytes[j]);
+    }
+    if (missing == 0) return hipSuccess;
+    if (held > 0 && held + missing <= most) {
+        void* p = nullptr;
+        ctx->bt_more.reserve(ctx->bt_more.size() + 1);
+        size_t got = most - held;
+        if (hipMalloc(&p, got) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+            got = missing;
+            if (hipMalloc(&p, got) != hipSuccess) p = nullptr;
+        }
+        if (p) {
+            ctx->bt_more.emplace_back(p, got);
+            room.emplace_back(static_cast<uint8_t*>(p), got);
+            for (size_t j = 0; j < bytes.size(); ++j)
+                if (!at[j]) place(j);
+            return hipSuccess;
+        }
+        (void)hipGetLastError();
+    }
+    for (const auto& c : ctx->bt_more) (void)hipFree(c.first);
+    ctx->bt_more.clear();
+    void* base = nullptr;
+    hipError_t e = bt_reserve(ctx, 0, held > 0 ? std::max(all, most) : all, &base);
+    if (e != hipSuccess && held > 0) {
+        (void)hipGetLastError();
+        e = bt_reserve(ctx, 0, all, &base);
+    }
+    if (e != hipSuccess) return e;
+    room.assign(1, {static_cast<uint8_t*>(base), ctx->bt_bytes[0]});
+    for (size_t j = 0; j < bytes.size(); ++j) place(j);
     return hipSuccess;
 }
 
@@ -1678,7 +1747,15 @@ int CigarCall::setup() {
     HIPCHK(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
     // the state this context already holds counts as free
     for (int i = 0; i < 7; ++i) free_b += ctx->bt_bytes[i];
-    budget = ctx->cigar_budget > 0 ? ctx->cigar_budget : (int64_t)(0.5 * (double)free_b);
+    for (const auto& c : ctx->bt_more) free_b += c.second;
+    budget = ctx->cigar_budget;
+    if (budget == 0) {
+        // half of it; the line of the call before while free memory is about
+        // the same, so that the same batch asks for the same state again
+        budget = (int64_t)(0.5 * (double)free_b);
+        if (std::abs(ctx->bt_budget - budget) <= budget / 8) budget = ctx->bt_budget;
+        ctx->bt_budget = budget;
+    }
     sc2.assign((size_t)b->n, 0);
     done.assign((size_t)b->n, 0);
     scored.assign((size_t)b->n, 0);
@@ -1704,7 +1781,9 @@ int CigarCall::launch_bt(const Shape& sh, KArgs& a, int32_t W, const std::vector
     if (sh.ck) ++cg->checkpoint_launches; else ++cg->record_launches;
     cg->kernels |= tsu_host::kernel_bit(sh);
     void *rec = nullptr, *slo = nullptr, *soff = nullptr, *ckb = nullptr;
-    HIPCHK(bt_reserve(ctx, 0, (size_t)(recs * grid) * 4, &rec), "hipMalloc (records)");
+    std::vector<void*> at;
+    HIPCHK(bt_place(ctx, {(size_t)(recs * grid) * 4}, (size_t)budget, at), "hipMalloc (records)");
+    rec = at[0];
     if (!sh.pk) {  // records at a place that depends on the score: a table
         HIPCHK(bt_reserve(ctx, 1, (size_t)((int64_t)step_cap * grid) * 4, &slo), "hipMalloc (steps)");
         HIPCHK(bt_reserve(ctx, 2, (size_t)((int64_t)step_cap * grid) * 8, &soff), "hipMalloc (steps)");
@@ -2094,14 +2173,14 @@ int CigarCall::record_pass() {
         int64_t words = 0;
         while (last < fl.plans.size() && (last == first || 4 * (words + fl.plans[last]->state_words) <= budget))
             words += fl.plans[last++]->state_words;
-        void* base = nullptr;
-        HIPCHK(bt_reserve(ctx, 0, (size_t)words * 4, &base), "hipMalloc (records)");
+        std::vector<size_t> sizes;
+        std::vector<void*> places;
+        for (size_t j = first; j < last; ++j) sizes.push_back((size_t)fl.plans[j]->state_words * 4);
+        HIPCHK(bt_place(ctx, sizes, (size_t)budget, places), "hipMalloc (records)");
         double load[2] = {0, 0};
-        uint32_t* at = static_cast<uint32_t*>(base);
         for (size_t j = first; j < last; ++j) {
             RecordPlan& p = *fl.plans[j];
-            p.state = at;
-            at += p.state_words;
+            p.state = static_cast<uint32_t*>(places[j - first]);
             const int k = load[1] < load[0] ? 1 : 0;
             for (int32_t i : p.ids) load[k] += (double)b->pairs[(size_t)i].p_len * p.win;
             r = start_plan(p, streams[k]);

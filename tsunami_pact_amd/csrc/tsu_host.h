@@ -51,6 +51,8 @@ struct tsu_ctx {
     // second.  Released by tsu_set_cigar_memory and tsu_destroy.
     void* bt_buf[7] = {};
     size_t bt_bytes[7] = {};
+    std::vector<std::pair<void*, size_t>> bt_more;  // further buffers of records, beside the first of bt_buf
+    int64_t bt_budget = 0;              // the budget (by free memory) it was sized for
 };
 
 struct tsu_batch {
