@@ -17,7 +17,9 @@ read once, the wavefronts stay on chip).  "roofline_valu" prices the work
 with a fixed op model -- 11 int32 lane-ops per cell-triple (one I, D and M
 update) and 16 per 32-base extend compare, the counts taken from the oracle
 on the CPU sample -- against the chip's int32 VALU peak (256 CUs x 64 lanes
-x 2.4 GHz).
+x 2.4 GHz).  The 4/6/2 kernel holds offsets of up to 32,000 bases as exact
+16-bit integers, two cells per lane-op in its recurrences (scores are int32),
+so the fraction could pass 1.
 
 The CPU baseline is the oracle's exact WFA (C, OpenMP over pairs, every host
 thread), timed on the first pairs of the same workload, and its scores double

@@ -879,7 +879,7 @@ struct Bucket {
 };
 
 // Bucket bounds on max(p, t).
-// (16383: the longest sequence the doubled-offset 16-chunk kernel takes)
+// (32000: the longest sequence the packed kernel takes)
 const int32_t kBucketBounds[] = {128, 256, 512, 1024, 2048, 4096, 8192, 16383, 32000, 1 << 26};
 
 }  // namespace
@@ -984,12 +984,12 @@ static const tsu_tune_entry* tune_lookup(const tsu_ctx* ctx, int32_t bound) { re
 // request's latency (the two margins measured alike there, within noise).
 
 // Capacity a probed pair gets: the predicted range with the margin, rounded
-// to the window of the kernel that will take it (64..512 one wave, 1024 two
-// waves, 4096 / 8192 / 16384 the 16-chunk kernel), so pairs fall into a few
-// launch groups.  Beyond 16,384 diagonals only the LDS kernel with its ring
-// in device memory remains, several times slower per diagonal: a pair goes
-// there directly only when even its unmargined prediction is well beyond
-// 16,384, and otherwise tries the 16-chunk kernel's widest window first.
+// to the window of the kernel that will take it (64..1024 one wave, 4096 /
+// 8192 / 16384 / 24576 several), so pairs fall into a few launch groups.
+// Beyond the widest window only the LDS kernel with its ring in device memory
+// remains, several times slower per diagonal: a pair goes there directly only
+// when even its unmargined prediction is well beyond that window, and
+// otherwise tries it first.
 int32_t tsu_host::probe_capacity(const tsu_ctx* ctx, const tsu_pair& pr, int32_t progress, double margin) {
     const double s_end = (double)kProbeCap * (double)(pr.p_len + pr.t_len) / (double)std::max(progress, 1);
     const double need = std::min(2.0 * (s_end - ctx->os) / ctx->es + 3.0, 1e9);
@@ -1825,7 +1825,7 @@ int CigarCall::grow_runs(int64_t more) {
 }
 
 // Pairs wider than every register window (they overflowed the 16,384
-// diagonals of the 16-chunk kernel): one LDS-kernel launch over the whole
+// diagonals that the packed kernel records): one LDS-kernel launch over the whole
 // diagonal range of their lengths, records sized for the highest score the
 // lengths allow, when that fits the budget (a few long divergent pairs, each
 // alone on a CU: a score pass first would double their time).

@@ -3,8 +3,7 @@
 // The 2-piece step of wfa2p.hip (WFA2-lib's affine-2p one: five wavefronts
 // M, I1, D1, I2, D2) for small gap extensions after the gcd, E1 = e1 and
 // E2 = e2 fixed at compile time ((2, 1) holds WFA2-lib's default 2-piece
-// penalties 4/6/2 + 24/1), laid out as the 1-piece single-wave kernel
-// (wfa_reg1l.h): one wave64 per pair, a window of 64 C diagonals, chunk c of
+// penalties 4/6/2 + 24/1): one wave64 per pair, a window of 64 C diagonals, chunk c of
 // lane l holding diagonal kmin + 64 c + l, offsets kept doubled (the bit
 // position of a base in the packed words), the extend fused into the step.
 //
