@@ -291,15 +291,15 @@ void tsu_cigars_free(tsu_cigars* c);
  *   budget_bytes     device memory one launch may hold for backtrace state,
  *                    0 = half the free device memory
  * The backtrace state stays allocated in the context between calls (freeing
- * tens of GB of device memory can take a second) and grows when a launch
- * needs more; this call and tsu_destroy release it. */
+ * tens of GB of device memory can take seconds) and grows, within the budget,
+ * when a call needs more; this call and tsu_destroy release it. */
 #define TSU_CIGAR_AUTO         0
 #define TSU_CIGAR_RECORDS      1
 #define TSU_CIGAR_CHECKPOINTS  2
 int tsu_set_cigar_memory(tsu_ctx* ctx, int32_t mode, int32_t checkpoint_every, int64_t budget_bytes);
-/* Waves of one pair that synchronise with their neighbours (score-only and
- * CIGAR launches of 1,025-16,384 diagonals) poll a neighbour's progress word at
- * most this many times per score before the pair fails with TSU_EINTERNAL
+/* Waves of one pair that synchronise with their neighbours (4/6/2 launches of
+ * several waves per pair, scores and CIGARs) poll a neighbour's progress word at
+ * most this many times per wait before the pair fails with TSU_EINTERNAL
  * instead of waiting for ever; 0 restores the default (2^20 polls, far above
  * any legitimate wait).  No reference counterpart (the reference's kernel
  * has one warp per pair); for callers that want a tighter bound and for
