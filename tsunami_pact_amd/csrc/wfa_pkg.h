@@ -29,8 +29,9 @@
 // last.  The plain form, whose answer is theirs, gives such pairs to them.
 //
 // What bounds it: instruction issue and LDS reads per chunk and score (45
-// vector, 20 scalar and 11 LDS instructions; vector units 63% busy at 5/6/2)
-// with one gap piece; with two, whose ring is two to four times as large, the
+// vector, 20 scalar and 11 LDS instructions with expanded sequences; 0.89
+// vector instructions per CU-cycle at 5/6/2 with packed ones) with one gap
+// piece; with two, whose ring is two to four times as large, the
 // pairs that fit a CU (vector units 32% busy with two pairs, 4/6/2/24/1).  Copying slot by slot at the exchange took 3.0 ms where
 // copying ten slots per LDS instruction takes 2.2 (20,000 x 1,000 bp at 5%,
 // 5/6/2, 397 diagonals; now 2.07; the ring kernel 9.2).
