@@ -1,0 +1,85 @@
+"""CIGARs of the packed kernel (4/6/2) where its 16-bit records do not hold an
+extension's length (4,095 bases and more): such lengths are in a list keyed by
+score and diagonal.  CIGARs are compared with the oracle's."""
+import random
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print(f"\n[gpu] {msg}", flush=True)
+
+
+def seq(rng, n):
+    return "".join(rng.choice("ACGT") for _ in range(n))
+
+
+def other(rng, c):
+    return rng.choice([x for x in "ACGT" if x != c])
+
+
+def substituted(rng, s, *places):
+    for i in places:
+        s = s[:i] + other(rng, s[i]) + s[i + 1:]
+    return s
+
+
+def gap_or_mismatch_first(rng, gap, same, tail):
+    """A gap of `gap` bases and a mismatch in either order, the same cost: on
+    the end diagonal the gap's cell lies `same` bases further than the
+    mismatch's, and both run into one match of `tail` bases."""
+    head, a, w, end = seq(rng, 900), rng.choice("ACGT"), seq(rng, same), seq(rng, tail)
+    p = substituted(rng, head, 300, 600) + other(rng, a) + w + seq(rng, gap - same - 1) + other(rng, a) + w + end
+    return p, head + a + w + end
+
+
+def gap_at_repeat(rng, gap, tail):
+    """The same with a substitution before the gap's other end."""
+    t = seq(rng, 100 + tail)
+    p = (t[:100] + other(rng, t[100]) + t[101:110] + other(rng, t[110]) + seq(rng, gap - 11) + other(rng, t[100]) + t[101:])
+    return substituted(rng, p, 20, 60), t
+
+
+def check_cigars(aligner, oracle, pairs, entries=()):
+    want, ops, _ = oracle.wfa_batch(pairs, 4, 6, 2, cigar=True)
+    aligner.set_tune_table(list(entries))
+    try:
+        got, cig, t = aligner.align_cigar(aligner.batch(pairs))
+    finally:
+        aligner.set_tune_table([])
+    assert (got == want).all(), np.nonzero(got != want)[0][:5]
+    bad = [i for i in range(len(pairs)) if cig[i] != oracle.rle(ops[i])]
+    assert not bad, (len(bad), bad[:5], cig[bad[0]], oracle.rle(ops[bad[0]]))
+    return t
+
+
+@pytest.mark.parametrize("window", [128, 256, 512, 1024, 2048, 4096, 8192])
+def test_long_extensions_at_chunk_edges(aligner, oracle, window):
+    """End diagonals in and beside every copy of a neighbour's diagonals at the
+    first chunk edges on both sides of diagonal 0, in one wave and several."""
+    rng = random.Random(window)
+    pairs = []
+    for gap in [g for g in [*range(30, 70), *range(160, 180)] if g < window // 2 - 8]:
+        for p, t in (gap_or_mismatch_first(rng, gap, 4, 4596), gap_or_mismatch_first(rng, gap, 1 + gap % 6, 4200),
+                     gap_at_repeat(rng, gap, 5900)):
+            pairs += [(p, t), (t, p)]
+    say(f"CIGARs of {len(pairs)} pairs in {window} diagonals")
+    check_cigars(aligner, oracle, pairs, [{"waves_per_pair": 1, "capacity": window, "bucket_bound": 8192}])
+
+
+@pytest.mark.parametrize("edits", [40, 100])
+def test_window_widened_by_another_pair(aligner, oracle, edits):
+    """The pairs' own scores fit 128 diagonals, but a pair with more edits in
+    the call takes all to a window of several chunks."""
+    rng = random.Random(edits)
+    pairs = []
+    for gap in (50, 52, 53, 54):
+        for p, t in (gap_or_mismatch_first(rng, gap, 4, 4596), gap_at_repeat(rng, gap, 5900)):
+            pairs += [(p, t), (t, p)]
+    wide = seq(rng, 5000)
+    pairs.append((wide, substituted(rng, wide, *rng.sample(range(5000), edits))))
+    say(f"CIGARs of {len(pairs)} pairs, one with {edits} substitutions")
+    check_cigars(aligner, oracle, pairs)

@@ -660,9 +660,12 @@ __global__ __launch_bounds__(NW * 64, pk_waves_per_simd(NW, C, H, BT)) void wfa_
                     cmp.extend_more(M, lim[c], more, b, kb - HALO + OWN * (NW * c + w), lane);
                     if constexpr (BT) {  // lengths a record does not hold
                         len = pk_minu(pk_sub(M, before), kPkLong * 0x10001u);
+                        // (of own diagonals: a copy whose gap source lies beyond
+                        // the chunk starts lower and would list a longer one)
+                        const bool own = HALO == 0 || (lane >= HL && lane < 64 - HL);
 #pragma unroll 1
                         for (int half = 0; half < 2; ++half) {
-                            if (((len >> (16 * half)) & 0xffffu) < kPkLong || pk_get(before, half) < 0) continue;
+                            if (!own || ((len >> (16 * half)) & 0xffffu) < kPkLong || pk_get(before, half) < 0) continue;
                             const uint32_t e = (pk_sub(M, before) >> (16 * half)) & 0xffffu;
                             const int i = atomicAdd(X + L::LC, 1);
                             if (i >= kPackedLongWords / 3) continue;
