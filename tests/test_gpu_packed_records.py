@@ -83,3 +83,55 @@ def test_window_widened_by_another_pair(aligner, oracle, edits):
     pairs.append((wide, substituted(rng, wide, *rng.sample(range(5000), edits))))
     say(f"CIGARs of {len(pairs)} pairs, one with {edits} substitutions")
     check_cigars(aligner, oracle, pairs)
+
+
+def low_complexity(rng):
+    """Tracts of short periods, where cells of many diagonals extend by 4,095
+    bases and more."""
+    h, pairs = seq(rng, 10), []
+    for unit in (1, 5):
+        u, d, end = seq(rng, unit), [seq(rng, 100) for _ in range(4)], seq(rng, 4800)
+        tract = (u * 5000)[:5000]
+        pairs.append((d[0] + tract + d[1] + end, d[2] + tract + d[3] + end))
+    segments = ("A" * 4600 + "C") * 3
+    pairs.append((h + "C" + segments + h, h + "G" + "A" * 400 + segments + h))
+    pairs.append((h + "C" + "ACAC" * 3900, h + "G" + "ACAC" * 3960))
+    return pairs
+
+
+@pytest.mark.parametrize("window", [0, 1024, 4096, 8192, 16384])
+def test_many_long_extensions(aligner, oracle, window):
+    """Hundreds to thousands of listed extensions, the walk's own among the
+    last, beside ordinary pairs; windows by the library (0) and pinned."""
+    rng = random.Random(31)
+    pairs = [q for p, t in low_complexity(rng) for q in ((p, t), (t, p))]
+    for n in (900, 5000, 9000):
+        p = seq(rng, n)
+        pairs.append((p, substituted(rng, p, *rng.sample(range(n), n // 40))))
+    say(f"CIGARs of {len(pairs)} pairs, window {window}")
+    check_cigars(aligner, oracle, pairs,
+                 [{"waves_per_pair": 1, "capacity": window, "bucket_bound": b} for b in (8192, 16383)] if window else [])
+
+
+def test_more_long_extensions_than_the_list_holds(aligner, oracle):
+    """Three segments of a homopolymer and a gap of 500 in 1,024 diagonals: 2,409
+    listed extensions where one wave's 9 chunks have room for 2,304 (over 512
+    pairs, so a pair has one wave), and the walk needs the last.  Such a pair
+    is recorded with offsets; the call's other pairs stay where they were."""
+    rng = random.Random(47)
+    h, segments = seq(rng, 10), ("A" * 4900 + "C") * 3
+    pair = (h + "C" + segments + h, h + "G" + "A" * 500 + segments + h)
+    pairs = [pair, pair[::-1]]
+    for _ in range(520):
+        p = seq(rng, rng.randint(8200, 8300))
+        pairs.append((p, substituted(rng, p, *rng.sample(range(8000), 3))))
+    say(f"CIGARs of {len(pairs)} pairs in 1,024 diagonals")
+    t = check_cigars(aligner, oracle, pairs, [{"waves_per_pair": 1, "capacity": 1024, "bucket_bound": 16383}])
+    assert t["kernels"] == {"reg1", "lds"}
+    say("with checkpoints where records do not fit")
+    aligner.set_cigar_memory(aligner.CIGAR_AUTO, 0, 8 << 20)
+    try:
+        t = check_cigars(aligner, oracle, pairs[:2], [{"waves_per_pair": 1, "capacity": 1024, "bucket_bound": 16383}])
+    finally:
+        aligner.set_cigar_memory()
+    assert t["state_bytes"] <= 8 << 20

@@ -1701,6 +1701,7 @@ private:
     int record_pass();
     int wide_pass();
     int score_first_pass();
+    int record_scored(const std::vector<int32_t>& by_score);
     int two_piece_pass();
     int collect(tsu_cigars** out);
 
@@ -1722,7 +1723,8 @@ private:
     int64_t budget = 0;
     std::vector<int32_t> sc2;      // scores the backtrace launches returned
     std::vector<uint8_t> done;
-    std::vector<uint8_t> scored;   // scored by the probe: records from the score-first path
+    std::vector<uint8_t> scored;   // scored by the probe
+    std::vector<uint8_t> offsets;  // more long extensions than the packed kernel lists: recorded with offsets
     std::vector<int32_t> wide;     // pairs that overflowed the widest register window
     std::vector<int32_t> wide_now; // those of them in the launch beside the record launches
     std::vector<int32_t> order;    // pairs of the score-first path
@@ -1759,6 +1761,7 @@ int CigarCall::setup() {
     sc2.assign((size_t)b->n, 0);
     done.assign((size_t)b->n, 0);
     scored.assign((size_t)b->n, 0);
+    offsets.assign((size_t)b->n, 0);
     return TSU_OK;
 }
 
@@ -2069,7 +2072,7 @@ void CigarCall::plan_group(int32_t W, bool placed, std::vector<int32_t>& ids, st
     // the window's scores
     const int64_t resident = std::min<int64_t>((int64_t)per_cu * ctx->cu_count, (int64_t)ids.size());
     const int64_t step_bytes = 4 * (tsu_host::packed_records(sh, 1) - tsu_host::packed_records(sh, 0));
-    const int64_t fit = budget / 2 / (resident * step_bytes) - tsu_host::packed_steps(1);
+    const int64_t fit = (budget / 2 / resident - 4 * tsu_host::packed_records(sh, 0)) / step_bytes - tsu_host::packed_steps(1);
     const int64_t s_win = s_cap;
     if (fit < s_cap) {
         if (fit * 3 < s_cap) return;
@@ -2103,6 +2106,7 @@ int CigarCall::settle_plan(const RecordPlan& pl, std::vector<int32_t>& wider) {
         const int32_t v = sc2[(size_t)i];
         const bool over = v == TSU_EKOVERFLOW || (v == TSU_ECIGAR && pl.at_window);
         if (v >= 0) { scores[i] = v; done[(size_t)i] = 1; }
+        else if (v == tsu::kLongListFull) offsets[(size_t)i] = 1;
         else if (over && pl.win >= 16 * 1024) wide.push_back(i);
         else if (over) wider.push_back(i);
         else if (v != TSU_ECIGAR)  // its step bound was the budget's: score first
@@ -2291,15 +2295,32 @@ int CigarCall::score_first_pass() {
     for (int32_t i : order)
         if (scores[i] < 0) return fail(ctx, scores[i], "pair " + std::to_string(i) + ": " + tsu_strerror(scores[i]));
     tsu_host::order_desc(order, [&](int32_t i) -> int64_t { return scores[i]; });
-    // their runs go after what the record launches used
+    std::vector<int32_t> first, last;
+    for (int32_t i : order) (offsets[(size_t)i] ? last : first).push_back(i);
+    if (!first.empty()) {
+        r = record_scored(first);
+        if (r != TSU_OK) return r;
+    }
+    if (tsu_host::fixed_242(ctx)) {  // pairs whose long extensions are too many for the packed kernel's list
+        HIPCHK(hipMemcpy(sc2.data(), b->d_scores, (size_t)b->n * sizeof(int32_t), hipMemcpyDeviceToHost), "hipMemcpy D2H");
+        for (int32_t i : first)
+            if (sc2[(size_t)i] == tsu::kLongListFull) { offsets[(size_t)i] = 1; last.push_back(i); }
+        tsu_host::order_desc(last, [&](int32_t i) -> int64_t { return scores[i]; });
+    }
+    return last.empty() ? TSU_OK : record_scored(last);
+}
+
+// Record launches of pairs with their scores known (in falling order).
+int CigarCall::record_scored(const std::vector<int32_t>& by_score) {
+    // their runs go after what the launches before reserved
     int64_t more = 0;
-    for (int32_t i : order) more += 2ll * (scores[i] / ctx->g / unit) + 2;
-    r = grow_runs(more);
+    for (int32_t i : by_score) more += 2ll * (scores[i] / ctx->g / unit) + 2;
+    int r = grow_runs(more);
     if (r != TSU_OK) return r;
     // group pairs into launches of similar score so buffers fit the widest
     size_t pos = 0;
-    while (pos < order.size()) {
-        const int32_t s0 = scores[order[pos]] / ctx->g;  // widest in this group (sorted desc)
+    while (pos < by_score.size()) {
+        const int32_t s0 = scores[by_score[pos]] / ctx->g;  // widest in this group (sorted desc)
         int32_t max_len = 0;
         size_t end = pos;
         // all pairs with score within this group share W and buffers
@@ -2310,11 +2331,11 @@ int CigarCall::score_first_pass() {
         // changes: a few pairs that need the LDS kernel do not take the
         // register kernels' pairs with them
         int family = -1;
-        for (end = pos; end < order.size(); ++end) {
-            const tsu_pair& pr = b->pairs[(size_t)order[end]];
+        for (end = pos; end < by_score.size(); ++end) {
+            const tsu_pair& pr = b->pairs[(size_t)by_score[end]];
             const int32_t len = std::max(pr.p_len, pr.t_len);
-            const int32_t si = scores[order[end]] / ctx->g;
-            const int f = bt_family(ctx, std::max<int32_t>(capacity_for_score(ctx, si), 16), len);
+            const int32_t si = scores[by_score[end]] / ctx->g;
+            const int f = offsets[(size_t)by_score[end]] ? 0 : bt_family(ctx, std::max<int32_t>(capacity_for_score(ctx, si), 16), len);
             if (family < 0) family = f;
             else if (f != family) break;
             max_len = std::max(max_len, len);
@@ -2327,7 +2348,7 @@ int CigarCall::score_first_pass() {
         sh.fixed_242 = tsu_host::fixed_242(ctx);
         int64_t recs = 0;
         int32_t step_cap = steps;
-        if (use_packed_recorder(ctx, W, max_len, sh)) {
+        if (family > 0 && use_packed_recorder(ctx, W, max_len, sh)) {
             step_cap = tsu_host::packed_steps(s0);
             recs = tsu_host::packed_records(sh, step_cap);
         } else {
@@ -2367,7 +2388,7 @@ int CigarCall::score_first_pass() {
             per_wg = recs * 4 + (int64_t)step_cap * 12 + (int64_t)a.ck_cap * a.ck_bytes +
                      (sh.lds_ring ? 0 : tsu::ring_bytes(sh, W, ctx->rm, ctx->ri));
         }
-        std::vector<int32_t> ids(order.begin() + (ptrdiff_t)pos, order.begin() + (ptrdiff_t)end);
+        std::vector<int32_t> ids(by_score.begin() + (ptrdiff_t)pos, by_score.begin() + (ptrdiff_t)end);
         r = launch_bt(sh, a, W, ids, max_len, recs, step_cap, per_wg);
         if (r != TSU_OK) return r;
         pos = end;

@@ -154,7 +154,7 @@ bool use_packed_kernel(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& sh
 // scores up to s.
 inline int32_t packed_steps(int64_t s) { return (int32_t)(s + 2 + tsu::kPackedStep); }
 inline int64_t packed_records(const Shape& sh, int32_t steps) {
-    return (int64_t)steps * sh.nw * sh.reg_c * 64 + tsu::kPackedLongWords;
+    return (int64_t)steps * sh.nw * sh.reg_c * 64 + tsu::packed_long_words(sh.nw * sh.reg_c);
 }
 
 // Probe of the batched and served forms: the single-wave register kernel

@@ -99,12 +99,18 @@ struct Shape {
 };
 
 // Packed kernel: scores it computes between two exchanges (it may record
-// that many scores past the end), and the words behind a workgroup's records
-// that list extensions too long for one (three words each).
+// that many scores past the end).
 constexpr int kPackedStep = 6;
 // The 2-piece register kernel's last score: past it a pair overflows.
 constexpr int kP2RegMaxScore = 16000;
-constexpr int kPackedLongWords = 768;
+// Words behind a workgroup's records that list the extensions too long for
+// one (three words each): two entries per diagonal of the window's chunks.
+// Tracts of 5,000-15,000 bases of period 1 to 5 fill 0.5 to 2.4 per diagonal
+// that the pair reaches.
+constexpr int packed_long_words(int chunks) { return 3 * 2 * 128 * chunks; }
+// Status of a pair whose walk needed an extension that found no room there:
+// the host records it with a kernel that keeps offsets in its records.
+constexpr int32_t kLongListFull = -1001;
 // Packed kernel for any penalties: own diagonals of a chunk, and the chunks
 // of a window.
 constexpr int kPkgOwn = 128 - 2 * kPackedStep;

@@ -365,7 +365,9 @@ constexpr int kPkSpinCap = 1 << 20;
 //   bit 2   I[s+1][k+1] opens from M[s-3][k] rather than extending I[s][k]
 //   bit 3   D[s+1][k-1] opens from M[s-3][k] rather than extending D[s][k]
 //   bits 4-15  the extension's length; kPkLong and above: kPkLong, and the
-//           length in the list behind the records (score, diagonal, length)
+//           length in the list behind the records (score, diagonal, length;
+//           packed_long_words).  A walk that needs a length the full list had
+//           no room for ends with kLongListFull: another kernel records the pair
 // The walk arrives at a cell with its offset after extension, so the length
 // gives the offset before.  16 bits per cell are half the record traffic and
 // half the state of records that hold the offset itself.
@@ -436,10 +438,16 @@ __device__ __forceinline__ int pk_walk(const uint32_t* rec, const uint32_t* long
             if (!record(w.ss, w.k, r)) return TSU_EINTERNAL;
             int e = (int)(r >> 4);
             if (e == (int)kPkLong) {
-                int i = 0;
-                while (i < n_longs && !((int)longs[3 * i] == w.ss && (int)longs[3 * i + 1] == w.k)) ++i;
-                if (i >= n_longs) return TSU_ECIGAR;  // the list was too short
-                e = (int)longs[3 * i + 2];
+                // 64 entries of the list at a time
+                int at = -1;
+                for (int i0 = 0; i0 < n_longs && at < 0; i0 += 64) {
+                    const int i = i0 + lane;
+                    const bool hit = i < n_longs && (int)longs[3 * i] == w.ss && (int)longs[3 * i + 1] == w.k;
+                    const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
+                    if (m) at = i0 + (int)__builtin_ctzll(m);
+                }
+                if (at < 0) return kLongListFull;
+                e = __builtin_amdgcn_readfirstlane((int)longs[3 * at + 2]);
             }
             w.emit(0, e);
             w.off -= e; w.v = w.off - w.k; w.h = w.off;
@@ -502,7 +510,7 @@ __global__ __launch_bounds__(NW * 64, pk_waves_per_simd(NW, C, H, BT)) void wfa_
     uint32_t* longs = nullptr;
     if constexpr (BT) {
         rec = a.rec_g + (int64_t)blockIdx.x * a.rec_cap;
-        longs = rec + a.rec_cap - kPackedLongWords;
+        longs = rec + a.rec_cap - packed_long_words(NC);
     }
 
     for (int iter = 0;; ++iter) {
@@ -668,7 +676,7 @@ __global__ __launch_bounds__(NW * 64, pk_waves_per_simd(NW, C, H, BT)) void wfa_
                             if (!own || ((len >> (16 * half)) & 0xffffu) < kPkLong || pk_get(before, half) < 0) continue;
                             const uint32_t e = (pk_sub(M, before) >> (16 * half)) & 0xffffu;
                             const int i = atomicAdd(X + L::LC, 1);
-                            if (i >= kPackedLongWords / 3) continue;
+                            if (i >= packed_long_words(NC) / 3) continue;
                             longs[3 * i] = (uint32_t)s;
                             longs[3 * i + 1] = (uint32_t)(k0 + OWN * NW * c + half);
                             longs[3 * i + 2] = e;
@@ -882,7 +890,7 @@ __global__ __launch_bounds__(NW * 64, pk_waves_per_simd(NW, C, H, BT)) void wfa_
                 int64_t out_off = 0;
                 int32_t out_n = 0;
                 if (st == 0)
-                    st = pk_walk<NC, OWN, HL>(rec, longs, min(__builtin_amdgcn_readfirstlane(X[L::LC]), kPackedLongWords / 3), kb,
+                    st = pk_walk<NC, OWN, HL>(rec, longs, min(__builtin_amdgcn_readfirstlane(X[L::LC]), packed_long_words(NC) / 3), kb,
                                               s0, score, p, t, a, &out_off, &out_n);
                 if (lane == 0) {
                     a.run_off[pi] = out_off;
