@@ -915,22 +915,10 @@ int32_t tsu_host::initial_capacity(const tsu_ctx* ctx, int32_t bound) {
     return std::max<int32_t>(W, 16);
 }
 
-Shape tsu_host::batched_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, int nw_hint, int64_t n) {
-    if (ctx->two_piece) {  // the 2-piece kernels, fed from the queue
-        Shape s2{1, max_len <= 32000, true, false, true};
-        s2.two_piece = true;
-        s2.reg_c = tsu_host::reg2p_chunks(ctx, W, max_len);
-        s2.reg_e = 10 * ctx->es + ctx->e2s;
-        use_packed_any(ctx, W, max_len, s2, n);
-        return s2;
-    }
+// Persistent launch of the LDS kernel (its ring in HBM when LDS is too small).
+static Shape ring_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, int nw_hint) {
     Shape sh{nw_hint > 0 ? nw_hint : default_waves(W), max_len <= 32000, true, false, true};
     sh.fixed_242 = tsu_host::fixed_242(ctx);
-    // a tuned hint above 1 asks for the LDS kernel with that many waves
-    if (nw_hint <= 1) {
-        use_register_kernel(ctx, W, max_len, sh, n);
-        if (sh.reg_c) return sh;
-    }
     tsu_host::place_sequences(ctx, sh, max_len);
     KArgs a = base_args(ctx);
     a.W = W;
@@ -940,6 +928,25 @@ Shape tsu_host::batched_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, in
         if (nw_hint <= 0) sh.nw = 16;
     }
     return sh;
+}
+
+Shape tsu_host::batched_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, int nw_hint, int64_t n) {
+    if (ctx->two_piece) {  // the 2-piece kernels, fed from the queue
+        Shape s2{1, max_len <= 32000, true, false, true};
+        s2.two_piece = true;
+        s2.reg_c = tsu_host::reg2p_chunks(ctx, W, max_len);
+        s2.reg_e = 10 * ctx->es + ctx->e2s;
+        use_packed_any(ctx, W, max_len, s2, n);
+        return s2;
+    }
+    // a tuned hint above 1 asks for the LDS kernel with that many waves
+    if (nw_hint <= 1) {
+        Shape sh{nw_hint > 0 ? nw_hint : default_waves(W), max_len <= 32000, true, false, true};
+        sh.fixed_242 = tsu_host::fixed_242(ctx);
+        use_register_kernel(ctx, W, max_len, sh, n);
+        if (sh.reg_c) return sh;
+    }
+    return ring_shape(ctx, W, max_len, nw_hint);
 }
 
 int32_t tsu_host::tuned_capacity(const tsu_ctx* ctx, int32_t bound) {
@@ -1359,9 +1366,11 @@ extern "C" int tsu_align_batched_noalloc(tsu_ctx* ctx, const uint32_t* d_words, 
                                              : initial_capacity(ctx, std::min(tsu_host::bucket_bound(bi), max_len));
         const int nw_hint = te ? te->waves_per_pair : 0;
         int32_t* region = d_order + base[(size_t)bi];
+        int ring_waves = -1;  // >= 0: the packed kernel's overflows on the ring kernel, at the same capacity
         for (int attempt = 0; !todo.empty(); ++attempt) {
             W = std::min<int32_t>(W, tsu_host::capacity_max(ctx, max_len));
-            const Shape sh = batched_shape(ctx, W, max_len, attempt == 0 ? nw_hint : 0, (int64_t)todo.size());
+            const int hint = attempt == 0 ? nw_hint : 0;
+            const Shape sh = ring_waves >= 0 ? ring_shape(ctx, W, max_len, ring_waves) : batched_shape(ctx, W, max_len, hint, (int64_t)todo.size());
             // (beyond 16,384 diagonals with 4/6/2 too, though a window that
             // needs no ring in device memory exists: a documented bound)
             if (!sh.lds_ring || (sh.pk && sh.win > 16 * 1024)) {
@@ -1391,7 +1400,14 @@ extern "C" int tsu_align_batched_noalloc(tsu_ctx* ctx, const uint32_t* d_words, 
             if (!again.empty()) {
                 if (W >= tsu_host::capacity_max(ctx, max_len)) return overflow_at(ctx, W, max_len);
                 retried += (int)again.size();
-                W = tsu_host::next_capacity(ctx, W, max_len);
+                // the packed kernel for any penalties overflows when a cell
+                // comes to the window's edge, the ring kernel when the range
+                // passes it: where no wider capacity is left for them, such
+                // pairs get the ring kernel
+                const int32_t wider = tsu_host::next_capacity(ctx, W, max_len);
+                const bool last = sh.pk && !sh.fixed_242 && !batched_shape(ctx, wider, max_len, 0, (int64_t)again.size()).lds_ring;
+                ring_waves = last ? hint : -1;
+                if (!last) W = wider;
             }
             todo.swap(again);
         }
