@@ -2110,8 +2110,10 @@ void CigarCall::plan_group(int32_t W, bool placed, std::vector<int32_t>& ids, st
     pl.grid = bt_grid(sh, a, (int64_t)pl.ids.size(), per_wg);
     if (pl.grid <= 0) { ids = std::move(pl.ids); return; }
     // (at least what one pair takes in twice as many diagonals, for the pairs
-    // that overflow: about twice the chunks for twice the scores)
-    pl.state_words = (recs * (win < 16 * 1024 ? std::max<int64_t>(pl.grid, 5) : pl.grid) + 63) / 64 * 64;
+    // that overflow: about twice the chunks for twice the scores; a quarter of
+    // the budget at most, else they are scored first)
+    const int64_t again = win < 16 * 1024 ? std::min<int64_t>(5 * recs, budget / 4 / 4) : 0;
+    pl.state_words = (std::max(recs * pl.grid, again) + 63) / 64 * 64;
     plans.push_back(std::move(pl));
 }
 
@@ -2148,7 +2150,7 @@ int CigarCall::start_plan(RecordPlan& pl, hipStream_t stream) {
                          pl.e0, pl.e1, none, &launched);
     if (r != TSU_OK) return r;
     if (!launched) return fail(ctx, TSU_EINTERNAL, "empty record launch");
-    cg->state_bytes = std::max(cg->state_bytes, pl.per_wg * pl.grid);
+    cg->state_bytes = std::max(cg->state_bytes, 4 * pl.state_words);
     ++cg->record_launches;
     cg->kernels |= tsu_host::kernel_bit(pl.sh);
     ++launches;
