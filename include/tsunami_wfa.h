@@ -291,8 +291,10 @@ void tsu_cigars_free(tsu_cigars* c);
  *   budget_bytes     device memory one launch may hold for backtrace state,
  *                    0 = half the free device memory
  * The backtrace state stays allocated in the context between calls (freeing
- * tens of GB of device memory can take seconds) and grows, within the budget,
- * when a call needs more; this call and tsu_destroy release it. */
+ * tens of GB of device memory can take seconds).  A call that needs more adds
+ * what it misses or as much as is held, whichever is more, within the budget;
+ * this call and tsu_destroy release it all.  A program that shares the device
+ * sets a budget, or calls this after its largest batch. */
 #define TSU_CIGAR_AUTO         0
 #define TSU_CIGAR_RECORDS      1
 #define TSU_CIGAR_CHECKPOINTS  2

@@ -50,3 +50,27 @@ def test_records_stay_within_the_budget(tsu, oracle, n, length, err, budget_mib)
         assert held <= (budget_mib << 20) + SLACK
     finally:
         a.close()
+
+
+def test_a_larger_call_grows_to_twice_what_it_needs_at_most(tsu, oracle):
+    """A small call, a larger one, the same again: the second adds at most as
+    much as is held or missing, the third nothing; set_cigar_memory gives all
+    back."""
+    small = tsu.Dataset.generate(60, seed=SEED + 1, len_min=1000, err_min=0.1)
+    large = tsu.Dataset.generate(120, seed=SEED + 2, len_min=3000, err_min=0.1)
+    a = tsu.Aligner(4, 6, 2)
+    try:
+        before = used(tsu)
+        t1 = check(a, oracle, small)
+        first = used(tsu) - before
+        t2 = check(a, oracle, large)
+        second = used(tsu) - before
+        say(f"held {first / 2**30:.2f} GiB, then {second / 2**30:.2f}; states {t1['state_bytes']}, {t2['state_bytes']}")
+        need = t2["state_bytes"] * t2["record_launches"]
+        assert second <= 2 * max(first, need) + SLACK
+        check(a, oracle, large)
+        assert used(tsu) - before <= second + SLACK
+        a.set_cigar_memory()
+        assert used(tsu) - before <= SLACK + (64 << 20)
+    finally:
+        a.close()

@@ -202,10 +202,10 @@ static hipError_t bt_reserve(tsu_ctx* ctx, int i, size_t bytes, void** p) {
 // Room for records of the given sizes, each in one piece, in the buffers the
 // context holds (buffer 0 and bt_more).  The first is as large as the first
 // call needs.  Getting and giving back tens of GB takes seconds (77 GB of
-// written memory: 8 s), so a call that needs more adds a second one with all
-// that is left of `most` (the budget), and only if that does not do either
-// does one buffer take their place.  The launches that used them have
-// completed.
+// written memory: 8 s), so a call that needs more adds a buffer as large as
+// what is held already, or as what is missing, within `most` (the budget), and
+// only if that does not do does one buffer take their place.  The launches
+// that used them have completed.
 static hipError_t bt_place(tsu_ctx* ctx, const std::vector<size_t>& bytes, size_t most, std::vector<void*>& at) {
     auto round = [](size_t n) { return (n + 255) & ~(size_t)255; };
     std::vector<std::pair<uint8_t*, size_t>> room;  // what is left of each buffer
@@ -235,7 +235,7 @@ static hipError_t bt_place(tsu_ctx* ctx, const std::vector<size_t>& bytes, size_
     if (held > 0 && held + missing <= most) {
         void* p = nullptr;
         ctx->bt_more.reserve(ctx->bt_more.size() + 1);
-        size_t got = most - held;
+        size_t got = std::min(most - held, std::max(missing, held));
         if (hipMalloc(&p, got) != hipSuccess) {
             (void)hipGetLastError();
             p = nullptr;
@@ -254,7 +254,7 @@ static hipError_t bt_place(tsu_ctx* ctx, const std::vector<size_t>& bytes, size_
     for (const auto& c : ctx->bt_more) (void)hipFree(c.first);
     ctx->bt_more.clear();
     void* base = nullptr;
-    hipError_t e = bt_reserve(ctx, 0, held > 0 ? std::max(all, most) : all, &base);
+    hipError_t e = bt_reserve(ctx, 0, std::max(all, std::min(most, 2 * held)), &base);
     if (e != hipSuccess && held > 0) {
         (void)hipGetLastError();
         e = bt_reserve(ctx, 0, all, &base);
