@@ -135,3 +135,14 @@ def test_more_long_extensions_than_the_list_holds(aligner, oracle):
     finally:
         aligner.set_cigar_memory()
     assert t["state_bytes"] <= 8 << 20
+
+
+def test_scored_pairs_of_the_widest_window(aligner, oracle):
+    """Unrelated pairs of 7,000 bases (8,193 to 16,384 diagonals), scored first
+    since their bucket is tuned to the LDS kernel: recorded by the packed
+    kernel's widest window."""
+    rng = random.Random(7)
+    pairs = [(seq(rng, 7000), seq(rng, 7000 - 40 * i)) for i in range(3)]
+    say("CIGARs of 3 unrelated pairs, scored first")
+    t = check_cigars(aligner, oracle, pairs, [{"waves_per_pair": 4, "capacity": 0, "bucket_bound": 8192}])
+    assert t["kernels"] == {"ml16"}, t["kernels"]

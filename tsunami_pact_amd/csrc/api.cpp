@@ -1603,6 +1603,7 @@ bool use_packed_recorder(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape& 
 // for the LDS kernel.
 int bt_family(const tsu_ctx* ctx, int32_t W, int32_t len) {
     Shape sh{1, true, true, true, true};
+    sh.fixed_242 = tsu_host::fixed_242(ctx);  // (the LDS its kernel takes depends on it)
     return use_packed_recorder(ctx, W, len, sh) ? std::max(sh.win, 1024) : 0;
 }
 
@@ -2002,24 +2003,9 @@ int CigarCall::plan_records(std::vector<RecordPlan>& plans, int64_t& runs_need) 
         }
         for (auto& kv : by) groups.push_back(Group{kv.first.second, true, std::move(kv.second)});
     }
-    // the groups of the 16-wave window share one launch: a pair fills a CU
-    // in either, and one launch leaves one tail instead of one per bucket
-    {
-        Group merged{0, false, {}};
-        std::vector<Group> rest;
-        for (Group& g : groups) {
-            int32_t ml = 0;
-            for (int32_t i : g.ids) ml = std::max(ml, std::max(b->pairs[(size_t)i].p_len, b->pairs[(size_t)i].t_len));
-            if (bt_family(ctx, std::min<int32_t>(g.W, capacity_full(ml, ml)), ml) == 16 * 1024) {
-                merged.W = std::max(merged.W, g.W);
-                merged.ids.insert(merged.ids.end(), g.ids.begin(), g.ids.end());
-            } else {
-                rest.push_back(std::move(g));
-            }
-        }
-        if (!merged.ids.empty()) rest.push_back(std::move(merged));
-        groups.swap(rest);
-    }
+    // (The buckets' groups of the 16-wave window stay launches of their own:
+    // as one launch 131 against 99 ms for 5,000 pairs of 100-20,000 bp, 322
+    // against 302 for 50,000; 22.2 against 23.5 for 4,000 of up to 10,000.)
     for (Group& g : groups) plan_group(g.W, g.placed, g.ids, plans, runs_need);
     // the pairs the probe finished, at their own scores (those the one-wave
     // recorder does not take are left to the score-first path)
