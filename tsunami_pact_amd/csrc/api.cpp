@@ -2148,9 +2148,12 @@ int CigarCall::start_plan(RecordPlan& pl, hipStream_t stream) {
 // persistent launch keeps its CUs until its queue drains, and the next
 // launches' workgroups take what it leaves, so the tails overlap (one launch
 // after another, each was waited for).  A pair that overflows its window is
-// recorded in twice as many diagonals behind the launch that found it.  Once
-// the launches of the widest window are done, the pairs wider than that run
-// on a third stream.
+// recorded in twice as many diagonals behind the launch that found it, in that
+// launch's state; where the pairs that did would fill more than twice that
+// state, after the launches in flight, in state of their own (3,000 unrelated
+// pairs of 500 bp 11.2 -> 2.8 ms, 2,000 of 1,000 bp 22.5 -> 5.9).  Once the
+// launches of the widest window are done, the pairs wider than that run on a
+// third stream.
 int CigarCall::record_pass() {
     std::vector<RecordPlan> planned;
     int64_t runs_need = 0;
@@ -2175,6 +2178,8 @@ int CigarCall::record_pass() {
     }
     hipStream_t streams[2] = {ctx->stream, ctx->stream3};
     bool wide_tried = false;
+    std::vector<std::unique_ptr<RecordPlan>> later;  // record again, after the launches in flight
+    int64_t later_runs = 0;
     for (size_t first = 0; first < fl.plans.size();) {
         // the launches that fit the budget together
         size_t last = first;
@@ -2212,18 +2217,25 @@ int CigarCall::record_pass() {
                 std::vector<int32_t> wider;
                 r = settle_plan(p, wider);
                 if (r != TSU_OK) return r;
-                // wider, on the same stream, in the state this launch leaves
+                // wider, on the same stream, in the state this launch leaves;
+                // where that is less than half of what they fill, later
                 std::vector<RecordPlan> next;
-                int64_t unused = 0;
-                if (!wider.empty()) plan_group(2 * p.win, false, wider, next, unused);
+                int64_t need = 0;
+                if (!wider.empty()) plan_group(2 * p.win, false, wider, next, need);
+                std::unique_ptr<RecordPlan> n;
                 if (!next.empty()) {
-                    const int64_t room = p.state_words / next[0].recs;
-                    next[0].grid = std::min(next[0].grid, room);
-                }
-                if (!next.empty() && next[0].grid > 0) {
-                    auto n = std::make_unique<RecordPlan>(std::move(next[0]));
+                    n = std::make_unique<RecordPlan>(std::move(next[0]));
                     n->d_ids = p.d_ids;
                     n->counter = p.counter;
+                    const int64_t room = p.state_words / n->recs;
+                    if (2 * room < n->grid) {
+                        later.push_back(std::move(n));
+                        later_runs += need;
+                    } else {
+                        n->grid = std::min(n->grid, room);
+                    }
+                }
+                if (n) {
                     n->state = p.state;
                     n->state_words = p.state_words;
                     std::swap(n->e0, p.e0);
@@ -2238,7 +2250,7 @@ int CigarCall::record_pass() {
                 }
             }
             // pairs wider than every window, once no launch can add to them
-            bool all_wide = last == fl.plans.size();
+            bool all_wide = last == fl.plans.size() && later.empty();
             for (const auto& p : fl.plans) all_wide = all_wide && (p->finished || p->win < 16 * 1024);
             if (all_wide && !wide.empty() && !wide_tried) {
                 wide_tried = true;
@@ -2252,6 +2264,17 @@ int CigarCall::record_pass() {
             if (!progressed) std::this_thread::sleep_for(std::chrono::microseconds(50));
         }
         first = last;
+        if (later.empty()) continue;
+        // most of a launch's pairs overflowed: their runs may be longer than
+        // was set aside (the wide launch, where it runs, holds the pool)
+        if (!wide_async.launched) {
+            r = grow_runs(later_runs);
+            if (r != TSU_OK) return r;
+        }
+        std::stable_sort(later.begin(), later.end(), [](const auto& x, const auto& y) { return x->win > y->win; });
+        for (auto& p : later) fl.plans.push_back(std::move(p));
+        later.clear();
+        later_runs = 0;
     }
     if (fl.plans.empty() && !wide.empty()) return TSU_OK;  // the wide pass runs them
     if (wide_async.launched) {
