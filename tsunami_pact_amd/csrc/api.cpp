@@ -2354,9 +2354,20 @@ int CigarCall::record_scored(const std::vector<int32_t>& by_score) {
         const int32_t W = std::max<int32_t>(capacity_for_score(ctx, s0), 16);
         const int32_t steps = s0 + 2;
         KArgs a = base_args(ctx);
+        // records of the LDS kernel up to s0
+        int64_t lds_recs = 64;
+        for (int64_t s = 0; s <= s0; ++s)
+            lds_recs += std::min<int64_t>(W, 2 * (std::max<int64_t>(0, s - ctx->os) / ctx->es + 2) + 1);
         // the group ends where the kernel family of a pair's own capacity
         // changes: a few pairs that need the LDS kernel do not take the
-        // register kernels' pairs with them
+        // register kernels' pairs with them.  But a pair of the packed
+        // kernel's widest window fills a CU in either, and joins an LDS launch
+        // that leaves CUs idle sooner than wait for its longest pair (50,000
+        // pairs of 100-20,000 bp, two that need the LDS kernel and 107 of the
+        // widest window: 314 ms a call apart, 300 together).
+        auto joins = [&](int f, int64_t n) {
+            return f == 16 * 1024 && n < ctx->cu_count && 4 * lds_recs * (n + 1) <= budget;
+        };
         int family = -1;
         for (end = pos; end < by_score.size(); ++end) {
             const tsu_pair& pr = b->pairs[(size_t)by_score[end]];
@@ -2364,7 +2375,7 @@ int CigarCall::record_scored(const std::vector<int32_t>& by_score) {
             const int32_t si = scores[by_score[end]] / ctx->g;
             const int f = offsets[(size_t)by_score[end]] ? 0 : bt_family(ctx, std::max<int32_t>(capacity_for_score(ctx, si), 16), len);
             if (family < 0) family = f;
-            else if (f != family) break;
+            else if (f != family && !(family == 0 && joins(f, (int64_t)(end - pos)))) break;
             max_len = std::max(max_len, len);
             if (end - pos >= 65536) break;
         }
@@ -2379,9 +2390,7 @@ int CigarCall::record_scored(const std::vector<int32_t>& by_score) {
             step_cap = tsu_host::packed_steps(s0);
             recs = tsu_host::packed_records(sh, step_cap);
         } else {
-            for (int64_t s = 0; s <= s0; ++s)
-                recs += std::min<int64_t>(W, 2 * (std::max<int64_t>(0, s - ctx->os) / ctx->es + 2) + 1);
-            recs += 64;
+            recs = lds_recs;
             tsu_host::place_sequences(ctx, sh, max_len);
             if (tsu::lds_bytes(sh, a) > ctx->max_lds) { sh.lds_ring = false; sh.nw = 16; }
         }
