@@ -144,7 +144,7 @@ extern "C" int tsu_create(tsu_ctx** out, int device, int32_t mismatch, int32_t g
         hipStreamCreateWithFlags(&ctx->stream3, hipStreamNonBlocking) != hipSuccess ||
         hipStreamCreateWithFlags(&ctx->stream_io, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess ||
-        hipMalloc(reinterpret_cast<void**>(&ctx->d_queue), 64 * sizeof(int32_t)) != hipSuccess) {
+        hipMalloc(reinterpret_cast<void**>(&ctx->d_queue), tsu_host::kQueueWords * sizeof(int32_t)) != hipSuccess) {
         tsu_destroy(ctx);
         return TSU_EHIP;
     }
@@ -1643,6 +1643,10 @@ struct RecordPlan {
     bool finished = false;
 };
 
+// Work counters of record launches in the context's queue words (word 0 is the
+// main stream's, 16 the wide launch's).
+constexpr size_t kRecordQueue = 20, kRecordCounters = tsu_host::kQueueWords - kRecordQueue;
+
 // Record launches in flight: on every return their streams are drained and
 // their events destroyed before the buffers they use are freed.
 struct RecordFlight {
@@ -2162,17 +2166,20 @@ int CigarCall::record_pass() {
     if (planned.empty() && wide.empty()) return TSU_OK;
     runs_cap = std::max<int64_t>(runs_need, 1);
     HIPCHK(d_runs.alloc((size_t)runs_cap), "hipMalloc (runs)");
-    DevBuf<int32_t> d_ids, d_counters;  // outlive the launches (declared before them)
-    HIPCHK(d_ids.alloc((size_t)std::max(b->n, 1)), "hipMalloc (order)");
-    HIPCHK(d_counters.alloc(std::max<size_t>(planned.size(), 1)), "hipMalloc (counters)");
+    // queue orders in the call's order array, work counters in the context's
+    // (a call of one pair took 245 us with both allocated, and polled, and
+    // 130 without)
+    DevBuf<int32_t> more_counters;  // outlives the launches (declared before them)
+    if (planned.size() > kRecordCounters) HIPCHK(more_counters.alloc(planned.size()), "hipMalloc (counters)");
+    int32_t* counters = more_counters.p ? more_counters.p : ctx->d_queue + kRecordQueue;
     // queued work (the probe's pairs, the counters) is done before other streams start
-    HIPCHK(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    if (planned.size() > 1) HIPCHK(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     RecordFlight fl;
     size_t ids_at = 0;
     for (size_t j = 0; j < planned.size(); ++j) {
         auto p = std::make_unique<RecordPlan>(std::move(planned[j]));
-        p->d_ids = d_ids.p + ids_at;
-        p->counter = d_counters.p + j;
+        p->d_ids = d_order.p + ids_at;
+        p->counter = counters + j;
         ids_at += p->ids.size();
         fl.plans.push_back(std::move(p));
     }
@@ -2199,8 +2206,13 @@ int CigarCall::record_pass() {
             r = start_plan(p, streams[k]);
             if (r != TSU_OK) return r;
         }
+        double waiting = now_ms();  // since the last launch ended
         for (size_t open = last - first; open > 0;) {
             bool progressed = false;
+            if (open == 1) {  // nothing else to look at meanwhile
+                for (size_t j = first; j < last; ++j)
+                    if (!fl.plans[j]->finished) HIPCHK(hipEventSynchronize(fl.plans[j]->e1), "hipEventSynchronize");
+            }
             for (size_t j = first; j < last; ++j) {
                 RecordPlan& p = *fl.plans[j];
                 if (p.finished) continue;
@@ -2261,7 +2273,8 @@ int CigarCall::record_pass() {
                     if (r != TSU_OK) return r;
                 }
             }
-            if (!progressed) std::this_thread::sleep_for(std::chrono::microseconds(50));
+            if (progressed) waiting = now_ms();
+            else if (now_ms() - waiting > 0.2) std::this_thread::sleep_for(std::chrono::microseconds(50));
         }
         first = last;
         if (later.empty()) continue;

@@ -141,6 +141,8 @@ int reg_waves(const tsu_ctx* ctx, int32_t W);
 // gcd, sequences up to 16000 bases, its M ring in LDS (0: the LDS-ring
 // 2-piece kernel).
 int reg2p_chunks(const tsu_ctx* ctx, int32_t W, int32_t max_len);
+// Words of a context's work counters (tsu_ctx::d_queue).
+constexpr size_t kQueueWords = 64;
 // Longest sequence the packed kernel takes: its offsets, and one past the
 // last one of a text with its padding, are exact in 16 bits.
 constexpr int32_t kPackedMaxLen = 32000;
