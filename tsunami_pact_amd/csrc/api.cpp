@@ -2088,12 +2088,11 @@ void CigarCall::plan_group(int32_t W, bool placed, std::vector<int32_t>& ids, st
     const int64_t recs = tsu_host::packed_records(sh, step_cap);
     const int64_t per_wg = recs * 4;
     // pairs of the widest window may also be walked by the launch for
-    // wider pairs, beside later launches: room for their whole bound; others
-    // by a launch in twice the window
+    // wider pairs, beside later launches: room for their whole bound
     for (int32_t i : ids) {
         const tsu_pair& pr = b->pairs[(size_t)i];
         const int64_t sb = score_bound(ctx, pr.p_len, pr.t_len);
-        runs_need += 2 * ((win >= 16 * 1024 ? sb : std::min<int64_t>(2 * step_cap, sb)) / unit) + 2;
+        runs_need += 2 * ((win >= 16 * 1024 ? sb : std::min<int64_t>(step_cap, sb)) / unit) + 2;
     }
     tsu_host::order_longest_first(ids, b->pairs.data());
     RecordPlan pl{std::move(ids), sh, a, W, max_len, step_cap, win, recs, per_wg, s_cap == s_win && s_win < s_len};
@@ -2164,7 +2163,10 @@ int CigarCall::record_pass() {
     int r = plan_records(planned, runs_need);
     if (r != TSU_OK) return r;
     if (planned.empty() && wide.empty()) return TSU_OK;
-    runs_cap = std::max<int64_t>(runs_need, 1);
+    // and a quarter more, for pairs recorded again (twice as much for all cost
+    // a call of 20,000 x 1,000 bp 0.2 of 1.9 ms)
+    int64_t runs_spare = runs_need / 4;
+    runs_cap = std::max<int64_t>(runs_need + runs_spare, 1);
     HIPCHK(d_runs.alloc((size_t)runs_cap), "hipMalloc (runs)");
     // queue orders in the call's order array, work counters in the context's
     // (a call of one pair took 245 us with both allocated, and polled, and
@@ -2230,7 +2232,8 @@ int CigarCall::record_pass() {
                 r = settle_plan(p, wider);
                 if (r != TSU_OK) return r;
                 // wider, on the same stream, in the state this launch leaves;
-                // where that is less than half of what they fill, later
+                // where that is less than half of what they fill, or the run
+                // words set aside are too few, later
                 std::vector<RecordPlan> next;
                 int64_t need = 0;
                 if (!wider.empty()) plan_group(2 * p.win, false, wider, next, need);
@@ -2240,11 +2243,12 @@ int CigarCall::record_pass() {
                     n->d_ids = p.d_ids;
                     n->counter = p.counter;
                     const int64_t room = p.state_words / n->recs;
-                    if (2 * room < n->grid) {
+                    if (2 * room < n->grid || need > runs_spare) {
                         later.push_back(std::move(n));
                         later_runs += need;
                     } else {
                         n->grid = std::min(n->grid, room);
+                        runs_spare -= need;
                     }
                 }
                 if (n) {
@@ -2278,7 +2282,7 @@ int CigarCall::record_pass() {
         }
         first = last;
         if (later.empty()) continue;
-        // most of a launch's pairs overflowed: their runs may be longer than
+        // many of a launch's pairs overflowed: their runs may be longer than
         // was set aside (the wide launch, where it runs, holds the pool)
         if (!wide_async.launched) {
             r = grow_runs(later_runs);
