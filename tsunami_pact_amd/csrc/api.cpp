@@ -663,16 +663,19 @@ static bool use_packed_any(const tsu_ctx* ctx, int32_t W, int32_t max_len, Shape
     if (tsu_host::fixed_242(ctx) || sh.bt || max_len > tsu_host::kPackedMaxLen) return false;
     if (ctx->os < 1 || (ctx->two_piece && ctx->o2s < 1)) return false;
     if (sh.reg_c && (sh.reg_c < 8 || (sh.reg_c == 8 && n > 8 * ctx->cu_count))) return false;
-    // with two pieces the widest capacity may be narrower than a pair needs,
-    // and the packed kernel reports such a pair a score early
-    if (ctx->two_piece && sh.queue && W < capacity_full(max_len, max_len) && W >= tsu_host::capacity_max(ctx, max_len)) return false;
     KArgs a = base_args(ctx);
     a.W = W;
     a.seq_words = seq_words_for(ctx, max_len);
     if (tsu::lds_bytes(sh, a) > ctx->max_lds) return false;
     Shape r = sh;
     r.pk = true;
-    r.win = sh.reg_c ? 64 * sh.reg_c : W;
+    // in place of the ring kernel, the capacity and that kernel's answer.  In
+    // place of the register kernel, its window and answer: what it and, for
+    // pairs that overflow there, the ring kernel at the capacity take between
+    // them is the ring kernel's where the window is as wide (or one wider)
+    const int32_t window = 64 * sh.reg_c;
+    r.pass = W >= window - 1;
+    r.win = r.pass ? W : window;
     r.reg_e = sh.reg_c ? sh.reg_e : 0;
     const int chunks = tsu::pkg_chunks(r.win);
     r.nw = chunks > 1 ? 2 : 1;
@@ -791,22 +794,20 @@ extern "C" int tsu_align_plain(tsu_ctx* ctx, tsu_batch* b, int32_t wf_length, in
     }
     int launches = 1;
     const bool clean = lowest >= 0;
-    if (!clean && (sh.two_piece ? sh.reg_c > 0 : sh.pk && !sh.fixed_242)) {
-        // the 2-piece register kernel stops past its score limit with an
-        // overflow status, and the packed kernel for any penalties when a
-        // cell comes to the window's edge: such pairs get the ring kernel at
-        // the same capacity, so whether a pair fits depends on the capacity
-        // and on neither (the re-run's launch counts in the wall time)
-        Shape s2{sh.two_piece ? 1 : default_waves(W), b->max_len <= 32000, true, false, true};
-        s2.two_piece = sh.two_piece;
-        s2.reg_e = sh.reg_e;
-        if (sh.pk) s2.reg_c = tsu_host::reg2p_chunks(ctx, W, b->max_len);
-        for (;;) {
-            const double r0 = now_ms();
-            std::vector<int32_t> again;
-            for (int32_t i = 0; i < b->n; ++i)
-                if (scores[i] == TSU_EKOVERFLOW) again.push_back(i);
-            if (again.empty()) break;
+    if (!clean && sh.two_piece && sh.reg_c > 0) {
+        // the 2-piece register kernel stops at the window's edge and past its
+        // score limit (the packed kernel in its place reports the latter):
+        // such pairs get the ring kernel at the same capacity, so whether a
+        // pair fits depends on the capacity and on neither (the re-run's
+        // launch counts in the wall time)
+        const double r0 = now_ms();
+        const int32_t open = sh.pk ? tsu::kScoreLimit : TSU_EKOVERFLOW;
+        std::vector<int32_t> again;
+        for (int32_t i = 0; i < b->n; ++i)
+            if (scores[i] == open) again.push_back(i);
+        if (!again.empty()) {
+            Shape s2{1, b->max_len <= 32000, true, false, true};
+            s2.two_piece = true;
             DevBuf<int32_t> d_order;
             HIPCHK(d_order.alloc(again.size()), "hipMalloc (order)");
             HIPCHK(hipMemcpy(d_order.p, again.data(), again.size() * sizeof(int32_t), hipMemcpyHostToDevice), "hipMemcpy (order)");
@@ -820,8 +821,6 @@ extern "C" int tsu_align_plain(tsu_ctx* ctx, tsu_batch* b, int32_t wf_length, in
             r = copy_to_host(ctx, scores, b->d_scores, (size_t)b->n * sizeof(int32_t));
             if (r != TSU_OK) return r;
             d2h += now_ms() - d0;
-            if (s2.reg_c == 0) break;
-            s2.reg_c = 0;
         }
     }
     if (t) {
@@ -915,21 +914,6 @@ int32_t tsu_host::initial_capacity(const tsu_ctx* ctx, int32_t bound) {
     return std::max<int32_t>(W, 16);
 }
 
-// Persistent launch of the LDS kernel (its ring in HBM when LDS is too small).
-static Shape ring_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, int nw_hint) {
-    Shape sh{nw_hint > 0 ? nw_hint : default_waves(W), max_len <= 32000, true, false, true};
-    sh.fixed_242 = tsu_host::fixed_242(ctx);
-    tsu_host::place_sequences(ctx, sh, max_len);
-    KArgs a = base_args(ctx);
-    a.W = W;
-    a.seq_words = seq_words_for(ctx, max_len);
-    if (tsu::lds_bytes(sh, a) > ctx->max_lds) {
-        sh.lds_ring = false;
-        if (nw_hint <= 0) sh.nw = 16;
-    }
-    return sh;
-}
-
 Shape tsu_host::batched_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, int nw_hint, int64_t n) {
     if (ctx->two_piece) {  // the 2-piece kernels, fed from the queue
         Shape s2{1, max_len <= 32000, true, false, true};
@@ -939,14 +923,22 @@ Shape tsu_host::batched_shape(const tsu_ctx* ctx, int32_t W, int32_t max_len, in
         use_packed_any(ctx, W, max_len, s2, n);
         return s2;
     }
+    Shape sh{nw_hint > 0 ? nw_hint : default_waves(W), max_len <= 32000, true, false, true};
+    sh.fixed_242 = tsu_host::fixed_242(ctx);
     // a tuned hint above 1 asks for the LDS kernel with that many waves
     if (nw_hint <= 1) {
-        Shape sh{nw_hint > 0 ? nw_hint : default_waves(W), max_len <= 32000, true, false, true};
-        sh.fixed_242 = tsu_host::fixed_242(ctx);
         use_register_kernel(ctx, W, max_len, sh, n);
         if (sh.reg_c) return sh;
     }
-    return ring_shape(ctx, W, max_len, nw_hint);
+    tsu_host::place_sequences(ctx, sh, max_len);
+    KArgs a = base_args(ctx);
+    a.W = W;
+    a.seq_words = seq_words_for(ctx, max_len);
+    if (tsu::lds_bytes(sh, a) > ctx->max_lds) {
+        sh.lds_ring = false;
+        if (nw_hint <= 0) sh.nw = 16;
+    }
+    return sh;
 }
 
 int32_t tsu_host::tuned_capacity(const tsu_ctx* ctx, int32_t bound) {
@@ -1366,11 +1358,9 @@ extern "C" int tsu_align_batched_noalloc(tsu_ctx* ctx, const uint32_t* d_words, 
                                              : initial_capacity(ctx, std::min(tsu_host::bucket_bound(bi), max_len));
         const int nw_hint = te ? te->waves_per_pair : 0;
         int32_t* region = d_order + base[(size_t)bi];
-        int ring_waves = -1;  // >= 0: the packed kernel's overflows on the ring kernel, at the same capacity
         for (int attempt = 0; !todo.empty(); ++attempt) {
             W = std::min<int32_t>(W, tsu_host::capacity_max(ctx, max_len));
-            const int hint = attempt == 0 ? nw_hint : 0;
-            const Shape sh = ring_waves >= 0 ? ring_shape(ctx, W, max_len, ring_waves) : batched_shape(ctx, W, max_len, hint, (int64_t)todo.size());
+            const Shape sh = batched_shape(ctx, W, max_len, attempt == 0 ? nw_hint : 0, (int64_t)todo.size());
             // (beyond 16,384 diagonals with 4/6/2 too, though a window that
             // needs no ring in device memory exists: a documented bound)
             if (!sh.lds_ring || (sh.pk && sh.win > 16 * 1024)) {
@@ -1400,14 +1390,7 @@ extern "C" int tsu_align_batched_noalloc(tsu_ctx* ctx, const uint32_t* d_words, 
             if (!again.empty()) {
                 if (W >= tsu_host::capacity_max(ctx, max_len)) return overflow_at(ctx, W, max_len);
                 retried += (int)again.size();
-                // the packed kernel for any penalties overflows when a cell
-                // comes to the window's edge, the ring kernel when the range
-                // passes it: where no wider capacity is left for them, such
-                // pairs get the ring kernel
-                const int32_t wider = tsu_host::next_capacity(ctx, W, max_len);
-                const bool last = sh.pk && !sh.fixed_242 && !batched_shape(ctx, wider, max_len, 0, (int64_t)again.size()).lds_ring;
-                ring_waves = last ? hint : -1;
-                if (!last) W = wider;
+                W = tsu_host::next_capacity(ctx, W, max_len);
             }
             todo.swap(again);
         }

@@ -74,6 +74,9 @@ struct KArgs {
     // probe_out, the largest h + v of its last scores
     int32_t probe_cap;
     int32_t* probe_out;
+    // packed kernel for any penalties: a pair overflows when its range leaves
+    // the window (else when a cell comes to its edge)
+    int32_t edge_pass;
 };
 
 // Score slot of a pair a probe launch stopped before its end (internal: the
@@ -95,6 +98,7 @@ struct Shape {
     bool pk = false;         // packed kernel (without fixed_242: for any penalties): nw waves of up to reg_c chunks of 128 diagonals, two per register
     bool expand = false;     // packed kernel with the sequences expanded in LDS
     int win = 0;             // packed kernels: the window's width in diagonals (KArgs::W of the launch)
+    bool pass = false;       // packed kernel for any penalties: KArgs::edge_pass
     int reg_e = 0;           // 2-piece register kernel (or the packed one in its place): 10 e1 + e2 after the gcd (11, 21 or 31)
 };
 
@@ -111,6 +115,10 @@ constexpr int packed_long_words(int chunks) { return 3 * 2 * 128 * chunks; }
 // Status of a pair whose walk needed an extension that found no room there:
 // the host records it with a kernel that keeps offsets in its records.
 constexpr int32_t kLongListFull = -1001;
+// Status of a pair of a plain launch that passed the score at which the
+// 2-piece register kernel, whose answer is wanted, stops: the ring kernel's
+// at the same capacity counts.
+constexpr int32_t kScoreLimit = -1002;
 // Packed kernel for any penalties: own diagonals of a chunk, and the chunks
 // of a window.
 constexpr int kPkgOwn = 128 - 2 * kPackedStep;

@@ -124,7 +124,10 @@ int launch_wfa(const Shape& sh, const KArgs& args, int64_t grid, void* stream) {
     KArgs a = args;
     if (sh.pk) {
         a.W = sh.win;  // the packed kernel's windows are wider than the capacity asked for
-        if (!sh.fixed_242) a.probe_cap = sh.reg_e ? kP2RegMaxScore : 0x3fffffff;  // wfa_pkg.h
+        if (!sh.fixed_242) {  // wfa_pkg.h
+            a.probe_cap = sh.pass ? 0x3fffffff : kP2RegMaxScore;
+            a.edge_pass = sh.pass;
+        }
     }
     KernelFn f = pick(sh);
     if (!f) return (int)hipErrorInvalidValue;

@@ -22,11 +22,18 @@
 //
 // Out-of-bounds I, D and M cells are NULL where they are computed, as in
 // wfa_pk.h (the oracle's orc_wfa_nulled: the same scores).  The window is
-// that of the ring or 2-piece register kernel it stands in for.  A non-NULL
-// cell on one of its edge diagonals (where that is no bound of the alignment)
-// ends the pair with TSU_EKOVERFLOW, at or before the score at which the
-// other kernel would; so does a score past probe_cap, the register kernel's
-// last.  The plain form, whose answer is theirs, gives such pairs to them.
+// that of the ring or 2-piece register kernel it stands in for, and so is the
+// answer whether a pair fits it (edges that are bounds of the alignment hold
+// nothing):
+//   edge_pass  the ring kernels': a pair overflows at the first score whose
+//          range leaves the window.  The first cell in bounds on an edge
+//          diagonal is a gap's (or M[0][0]), and where GI or GD of s holds one
+//          the range goes beyond at s + e: the end must be reached before the
+//          least of these (before o + e where diagonal 0 is an edge).
+//   else   the 2-piece register kernel's: at the first score with a cell in
+//          bounds on an edge diagonal, unless it ends there.  Past probe_cap,
+//          that kernel's last score, the ring kernel's answer at the capacity
+//          asked for counts; the plain form gives such pairs to it.
 //
 // What bounds it: instruction issue and LDS reads per chunk and score (45
 // vector, 20 scalar and 11 LDS instructions with expanded sequences; 0.89
@@ -41,6 +48,7 @@
 
 namespace tsu {
 
+constexpr int kPkEvPass = 2;  // the range leaves the window after this score (wfa_pk.h: the other events)
 constexpr int kPkgHl = kPkStep / 2;   // lanes of copies at each end
 constexpr uint32_t kPkgNone = ~0u;  // a lane that copies nothing
 constexpr int kPkgRenull = 8190;  // scores, a multiple of kPkStep: NULL grows by one per score
@@ -84,7 +92,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
     const int sw = (int)pk_packed_words((uint32_t)a.seq_words);
     const uint32_t tb = 2 * (hn + hp), pb = tb + 4u * (uint32_t)sw;
     uint32_t* sS = smem + tb / 4;
-    int32_t* X = reinterpret_cast<int32_t*>(sS + 2 * sw);  // [0] queue index, [1] first event
+    int32_t* X = reinterpret_cast<int32_t*>(sS + 2 * sw);  // [0] queue index, [1] first event, [2] edges
     uint32_t* ring = reinterpret_cast<uint32_t*>(X + 4);
     const uint32_t rb = tb + 8u * (uint32_t)sw + 16u;      // its byte address
     const bool lds_at_zero = (uint32_t)(uintptr_t)smem == 0u;
@@ -119,7 +127,13 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
         if constexpr (RG) {
             for (int i = tid; i < 2 * (E1 + E2) * NC * 2 * HL; i += NT) pk_st32(gx + 4u * (uint32_t)i, kPkNull);
         }
-        if (tid == 0) X[1] = kPkNoEvent;
+        if (tid == 0) {
+            // the event of a gap cell of piece 1 or 2 on an edge, less 4 s (in
+            // LDS: in registers it costs the score loop spills)
+            auto then = [&](int scores) -> int { return a.edge_pass ? 4 * (scores - 1) + kPkEvPass : kPkEvEdge; };
+            X[1] = W > 2 ? kPkNoEvent : then(P == 2 ? min(a.o + a.e, a.o2 + a.e2) : a.o + a.e);  // (diagonal 0 an edge)
+            X[2] = then(a.e) | (P == 2 ? then(a.e2) << 16 : 0);
+        }
         __syncthreads();
         if constexpr (H) {
             pk_expand(smem, hn, hp, sS, sw, tid, NT);
@@ -283,8 +297,9 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
                     const uint32_t u = __builtin_amdgcn_update_dpp(0u, v, 0x130, 0xF, 0xF, true);
                     return __builtin_amdgcn_alignbit(u, v, 16);
                 };
-                // Score s from the G slots it reads; put() gets their new values.
-                auto score = [&](int s, uint32_t i1, uint32_t d1, uint32_t i2, uint32_t d2, auto put) __attribute__((always_inline)) {
+                // Score s from the G slots it reads; put() gets their new
+                // values, now(i) gives one back (GI1, GD1, GI2, GD2).
+                auto score = [&](int s, uint32_t i1, uint32_t d1, uint32_t i2, uint32_t d2, auto put, auto now) __attribute__((always_inline)) {
                     const uint32_t mx = pk_ld32(A + qx), mo = pk_ld32(A + qo);
                     uint32_t mo2 = 0;
                     if constexpr (P == 2) mo2 = pk_ld32(A + qo2);
@@ -317,11 +332,23 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
                     const uint32_t more = f & PkCompare<H>::FULL;
                     if (pk_any(more)) cmp.extend_more(M, lim, more, pl, kb - kPkStep + OWN * j, lane);
                     pk_st32(A + qm, M);
-                    if (special && pk_any(pk_sub_sat(watch, pk_max(raw, M)) & 0x80008000u)) {
+                    if (__builtin_expect(special && pk_any(pk_sub_sat(watch, pk_max(raw, M)) & 0x80008000u), 0)) {
                         auto at = [&](uint32_t v, int place) -> int { return (int16_t)((uint32_t)__builtin_amdgcn_readlane((int)v, place >> 1) >> (16 * (place & 1))); };
                         if (at_end && at(M, ptp) >= t) ev = min(ev, 4 * s + kPkEvEnd);
-                        if (at_lo && at(raw, kPkStep) >= 0) ev = min(ev, 4 * s + kPkEvEdge);
-                        if (at_hi && at(raw, phi) >= 0) ev = min(ev, 4 * s + kPkEvEdge);
+                        const uint32_t adds = __builtin_amdgcn_readfirstlane((uint32_t)X[2]);
+                        auto edge = [&](int place, uint32_t g1, uint32_t g2) {
+                            if (at(g1, place) >= 0) ev = min(ev, 4 * s + (int)(adds & 0xffffu));
+                            if (P == 2 && at(g2, place) >= 0) ev = min(ev, 4 * s + (int)(adds >> 16));
+                        };
+                        // M stands for the piece that extends slower (what it
+                        // adds is no less than the other's); with W of 1 or 2,
+                        // which only queues take, a pair may go wider early
+                        if constexpr (RG) {  // (e2 = 1; a chunk has one edge at most)
+                            if (at_lo || at_hi) edge(at_lo ? kPkStep : phi, M, at_lo ? now(3) : now(2));
+                        } else {
+                            if (at_lo) edge(kPkStep, P == 1 ? M : now(1), now(3));
+                            if (at_hi) edge(phi, P == 1 ? M : now(0), now(2));
+                        }
                     }
                     qm = next(qm, Rb); qx = next(qx, Rb); qo = next(qo, Rb);
                     if constexpr (P == 2) qo2 = next(qo2, Rb);
@@ -332,7 +359,7 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
                         uint32_t &gi = G[i % E1], &gd = G[E1 + i % E1], &gi2r = G[2 * E1 + i % E2], &gd2r = G[2 * E1 + E2 + i % E2];
                         score(s0 + i, gi, gd, gi2r, gd2r, [&](uint32_t ni, uint32_t nd, uint32_t ni2, uint32_t nd2) __attribute__((always_inline)) {
                             gi = ni; gd = nd; gi2r = ni2; gd2r = nd2;
-                        });
+                        }, [&](int i) __attribute__((always_inline)) -> uint32_t { return i == 0 ? gi : i == 1 ? gd : i == 2 ? gi2r : gd2r; });
                     }
                     if (g_out) {
                         const uint32_t at = gx + 4u * (uint32_t)(j * 2 * HL + (lane < 32 ? lane - HL : lane - (64 - 2 * HL) + HL));
@@ -350,6 +377,8 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
                             pk_st32(ai1, ni);
                             pk_st32(ad1, nd);
                             if constexpr (P == 2) { pk_st32(ai2, ni2); pk_st32(ad2, nd2); }
+                        }, [&](int i) __attribute__((always_inline)) -> uint32_t {
+                            return P == 1 ? kPkNull : pk_ld32(i == 0 ? ai1 : i == 1 ? ad1 : i == 2 ? ai2 : ad2);
                         });
                         qg = next(qg, eb);
                         if constexpr (P == 2) qg2 = next(qg2, eb2);
@@ -365,7 +394,10 @@ __global__ __launch_bounds__(NW * 64) void wfa_pkg_kernel(KArgs a) {
             const int ev = X[1];
             int score = r;
             if (same) score = 0;
-            else if ((ev >> 2) <= s0) score = (ev & 3) == kPkEvEnd && (ev >> 2) <= a.probe_cap ? (ev >> 2) : TSU_EKOVERFLOW;
+            else if ((ev >> 2) <= s0) {
+                score = (ev & 3) == kPkEvEnd ? (ev >> 2) : TSU_EKOVERFLOW;
+                if ((ev >> 2) > a.probe_cap) score = QUEUE ? TSU_EKOVERFLOW : kScoreLimit;
+            }
             a.scores[pi] = !lds_at_zero ? TSU_EINTERNAL : score < 0 ? score : score * a.g;
         }
         __syncthreads();  // LDS reused by the next pair of this workgroup
