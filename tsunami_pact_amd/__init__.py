@@ -445,9 +445,9 @@ class Aligner:
                     "tsu_set_cigar_memory")
 
     def set_poll_limit(self, polls: int = 0) -> None:
-        """Polls of a neighbour's progress before a pair fails with
-        TSU_EINTERNAL (score-only launches of 1,025-16,384 diagonals); 0 =
-        the default."""
+        """Polls of a neighbour's progress per wait before a pair fails with
+        TSU_EINTERNAL (4/6/2 launches of several waves per pair, scores and
+        CIGARs); 0 = the default."""
         self._check(self._lib.tsu_set_poll_limit(self._h, polls), "tsu_set_poll_limit")
 
     def align_cigar(self, batch: Batch, strings=True, count_runs: bool = False):

@@ -1666,8 +1666,8 @@ struct WideAsync {
 };
 
 // One tsu_align_cigar call.  Three paths, each over the pairs the ones
-// before it left: record launches without a score pass (register kernels,
-// per length bucket at the batched form's capacity), one LDS-kernel launch
+// before it left: record launches without a score pass (packed kernel, per
+// length bucket at the batched form's capacity), one LDS-kernel launch
 // over the whole diagonal range for pairs wider than every register window,
 // and scores first (batched form) for the rest, which size the backtrace
 // state exactly.  The walks append their runs to one pool on the device.
@@ -1769,8 +1769,6 @@ int CigarCall::setup() {
     return TSU_OK;
 }
 
-// One backtrace launch of `ids` with `recs` record words and `step_cap`
-// scores of state per workgroup (per_wg bytes in all).
 // Workgroups of a backtrace launch of n pairs: every pair that fits on the
 // CUs at once, within the budget (0: the shape has no occupancy).
 int64_t CigarCall::bt_grid(const Shape& sh, const KArgs& a, int64_t n, int64_t per_wg) const {
@@ -1780,6 +1778,8 @@ int64_t CigarCall::bt_grid(const Shape& sh, const KArgs& a, int64_t n, int64_t p
     return std::max<int64_t>(1, std::min<int64_t>(grid, budget / std::max<int64_t>(per_wg, 1)));
 }
 
+// One backtrace launch of `ids` with `recs` record words and `step_cap`
+// scores of state per workgroup (per_wg bytes in all).
 int CigarCall::launch_bt(const Shape& sh, KArgs& a, int32_t W, const std::vector<int32_t>& ids, int32_t max_len,
                          int64_t recs, int32_t step_cap, int64_t per_wg) {
     const int64_t grid = bt_grid(sh, a, (int64_t)ids.size(), per_wg);
@@ -1913,17 +1913,19 @@ int CigarCall::launch_wide_async(WidePlan& wp, const std::vector<int32_t>& ids) 
 }
 
 // Record launches without a score pass, per length bucket of the batched
-// form at its capacity, where a register kernel records: the state is sized
+// form at its capacity, where the packed kernel records: the state is sized
 // for the highest score the window (or the lengths) allow.  A pair whose
-// window overflows, or whose score passes that step bound, is left to the
-// paths after.
+// window overflows is recorded again in twice the window (record_pass); one
+// whose score passes the budget's step bound, or with more long extensions
+// than the recorder lists, is left to the paths after.
 //
 // Buckets whose first window needs several waves are probed first, as in the
-// batched form: a pair the probe finished has its score, and its records come
-// from the score-first path's launches at its exact capacity; the others are
-// grouped by bucket and predicted window, so a low-error pair of 10 kbp
-// records in 4,096 diagonals (four waves, a quarter of the record state)
-// rather than its bucket's 16,384.
+// batched form: the pairs the probe finished have their scores and share one
+// launch sized for the highest of them (those longer than its narrow windows
+// take are left to the score-first path); the others are grouped by bucket
+// and predicted window, so a low-error pair of 10 kbp records in 4,096
+// diagonals (four waves, a quarter of the record state) rather than its
+// bucket's 16,384.
 int CigarCall::plan_records(std::vector<RecordPlan>& plans, int64_t& runs_need) {
     const int nb = tsu_host::bucket_count();
     // one pass for every pair's bucket and each bucket's count and longest
@@ -2366,7 +2368,7 @@ int CigarCall::record_scored(const std::vector<int32_t>& by_score) {
         // pairs of 100-20,000 bp, two that need the LDS kernel and 107 of the
         // widest window: 314 ms a call apart, 300 together).
         auto joins = [&](int f, int64_t n) {
-            return f == 16 * 1024 && n < ctx->cu_count && 4 * lds_recs * (n + 1) <= budget;
+            return f == 16 * 1024 && n < ctx->cu_count && 4 * lds_recs * (n + 1) <= budget / 2;
         };
         int family = -1;
         for (end = pos; end < by_score.size(); ++end) {

@@ -47,8 +47,8 @@ struct tsu_ctx {
     // backtrace state of tsu_align_cigar (records, step bounds, step offsets,
     // checkpoints; then records, step bounds and step offsets of the launch
     // on the second stream), kept between calls and grown when a launch
-    // needs more: freeing tens of GB of written device memory can take a
-    // second.  Released by tsu_set_cigar_memory and tsu_destroy.
+    // needs more: freeing tens of GB of written device memory can take
+    // seconds.  Released by tsu_set_cigar_memory and tsu_destroy.
     void* bt_buf[7] = {};
     size_t bt_bytes[7] = {};
     std::vector<std::pair<void*, size_t>> bt_more;  // further buffers of records, beside the first of bt_buf

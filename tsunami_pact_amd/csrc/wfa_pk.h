@@ -58,9 +58,11 @@
 // words, at 4.5 instead of 0.5 bytes of LDS per base of a pair.  The host
 // takes H where that leaves enough waves per CU.
 //
-// What bounds it: vector issue.  A chunk and score takes about 30 vector
-// instructions for 128 cells, where the kernels it replaced took 29-35 for
-// 64; with 4 waves per SIMD a CU issues 0.66 vector instructions per cycle
+// What bounds it: vector issue.  A chunk and score takes 29 vector
+// instructions for 128 cells where no cell is out of bounds or extends past
+// its first compare (37 counted over all of a 1,000 bp pair at 5%: those, the
+// exchanges and the setup), where the kernels it replaced took 29-35 for 64;
+// with 4 waves per SIMD a CU issues 0.66 vector instructions per cycle
 // (16 waves per pair) to 0.83 (8 waves), what is missing being LDS latency.
 // Measured, before (32-bit offsets in registers, older M scores in an LDS
 // ring, a wait per score) and after: 30,000 pairs of 100-20,000 bp at 1-15%,
